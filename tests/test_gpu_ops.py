@@ -467,6 +467,25 @@ def test_attention_f16_vs_oracle(ctx, B, ctxlen, H, HKV, HD, n_split):
         assert rel_l2(got[b], want) <= REL_L2, (b, rel_l2(got[b], want))
 
 
+@pytest.mark.parametrize("H,HKV,HD,n,n_split", [(40, 8, 128, 3900, 0), (40, 8, 128, 8100, 0), (10, 2, 64, 8100, 64),
+                                                (40, 8, 128, 8300, 61), (28, 4, 128, 8100, 64), (8, 8, 64, 8192, 33)])
+def test_attention_merges_every_split(ctx, H, HKV, HD, n, n_split):
+    """One query over more key splits than one batch of the merge's loads: 30 splits where 5 heads
+    share a KV head (3 or 6 thread sets), 32 elsewhere; every split's keys reach the output."""
+    rng = np.random.default_rng(n + n_split)
+    q8, sc, deq = q8_cache(rng, 1, HKV, n, HD)
+    v8, vsc, vdeq = q8_cache(rng, 1, HKV, n, HD)
+    q = rng.standard_normal((1, H * HD)).astype(np.float32)
+    scale = float(np.float32(1) / np.sqrt(np.float32(HD)))
+    out = ctx.alloc(q.nbytes)
+    ctx.attn_decode(ctx.to_device(q), 1, H, HKV, HD, ctx.to_device(q8), ctx.to_device(sc), ctx.to_device(v8),
+                    ctx.to_device(vsc), n, ctx.to_device(np.array([n], np.int32)), 1, scale, out, n_split=n_split)
+    kc = deq[0].transpose(1, 0, 2).reshape(n, HKV * HD)
+    vc = vdeq[0].transpose(1, 0, 2).reshape(n, HKV * HD)
+    want = oracle.attention(q[0], kc, vc, H, HKV, HD, n - 1, scale)
+    assert rel_l2(out.download(np.float32), want) <= 2e-5
+
+
 def test_attention_most_work_items_twice(ctx):
     """B * HKV = 4096 (the per-op entry point's limit) with 8 key splits each:
     every (query, KV head) merge counter counts 8 workgroups and its last one

@@ -430,7 +430,8 @@ __device__ inline void attn_merge(const AttnArgs &a, int b, int kvh, int n_split
     constexpr int NOUT = G * HD, NQ4 = NOUT / 4, NW = NT / 64;
     constexpr int SETS = NT / NQ4 < 1 ? 1 : (NT / NQ4 > NW ? NW : NT / NQ4);
     constexpr int PER = (NQ4 + NT - 1) / NT;  // quads a thread (SETS 1 with more quads than threads)
-    constexpr int MB = 32 / SETS;             // loads a thread per quad and batch: 32 splits a batch in all
+    constexpr int MB = 32 / SETS;             // loads a thread per quad and batch
+    constexpr int BATCH = SETS * MB;          // splits a batch: 32, or 30 where SETS (G 5: 3 or 6) does not divide 32
     constexpr int64_t grp = attn_group_floats(G, HD);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int set = SETS > 1 ? tid / NQ4 : 0, tq = SETS > 1 ? tid % NQ4 : tid;
@@ -468,7 +469,7 @@ __device__ inline void attn_merge(const AttnArgs &a, int b, int kvh, int n_split
 #pragma unroll
     for (int k = 0; k < PER; k++) acc[k] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (active) {
-        for (int s0 = 0; s0 < used; s0 += 32) {
+        for (int s0 = 0; s0 < used; s0 += BATCH) {
             if (s0) fetch(s0);
 #pragma unroll
             for (int k = 0; k < PER; k++) {
