@@ -167,19 +167,20 @@ __global__ __launch_bounds__(256) void k_act_half(const float *__restrict__ x, i
             const float4 v = value4(32 * c + 4 * k);
             const float f[4] = {v.x * scale, v.y * scale, v.z * scale, v.w * scale};
 #pragma unroll
-            for (int j = 0; j < 4; j += 2) {
-                const _Float16 h0 = (_Float16)f[j], h1 = (_Float16)f[j + 1];
-                const _Float16 l0 = (_Float16)(f[j] - (float)h0), l1 = (_Float16)(f[j + 1] - (float)h1);
-                hw[2 * k + j / 2] = __builtin_bit_cast(uint16_t, h0) | (uint32_t)__builtin_bit_cast(uint16_t, h1) << 16;
-                lw[2 * k + j / 2] = __builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
-                sum += f[j] + f[j + 1];
+            for (int j = 0; j < 2; j++) {  // values j and j + 2 of four a dword
+                const _Float16 h0 = (_Float16)f[j], h1 = (_Float16)f[j + 2];
+                const _Float16 l0 = (_Float16)(f[j] - (float)h0), l1 = (_Float16)(f[j + 2] - (float)h1);
+                hw[2 * k + j] = __builtin_bit_cast(uint16_t, h0) | (uint32_t)__builtin_bit_cast(uint16_t, h1) << 16;
+                lw[2 * k + j] = __builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
             }
+            sum += f[0] + f[1];
+            sum += f[2] + f[3];
         }
-        uint8_t *blk = o + (size_t)(c / 8) * 1024 + (c % 8) * 64;
+        uint8_t *blk = o + (size_t)(c / 8) * 1024 + hact_piece(c % 8, 0);
 #pragma unroll
         for (int k = 0; k < 4; k++) {
-            ((uint4 *)blk)[k] = make_uint4(hw[4 * k], hw[4 * k + 1], hw[4 * k + 2], hw[4 * k + 3]);
-            ((uint4 *)(blk + 512))[k] = make_uint4(lw[4 * k], lw[4 * k + 1], lw[4 * k + 2], lw[4 * k + 3]);
+            *(uint4 *)(blk + 256 * k) = make_uint4(hw[4 * k], hw[4 * k + 1], hw[4 * k + 2], hw[4 * k + 3]);
+            *(uint4 *)(blk + 256 * k + 64) = make_uint4(lw[4 * k], lw[4 * k + 1], lw[4 * k + 2], lw[4 * k + 3]);
         }
         const float xs = sum * (1.0f / 32);  // exact; keeps the sums in fp16 range
         const _Float16 xh = (_Float16)xs, xl = (_Float16)(xs - (float)xh);
@@ -247,22 +248,24 @@ __global__ __launch_bounds__(256) void k_act_half_reg(const float *__restrict__ 
         uint32_t hw[8], lw[8];
         float sum = 0.f;
 #pragma unroll
-        for (int j = 0; j < 16; j += 2) {
-            const float f0 = v[k][j] * scale, f1 = v[k][j + 1] * scale;
+        for (int j = 0; j < 16; j += 2) sum += v[k][j] * scale + v[k][j + 1] * scale;
+#pragma unroll
+        for (int j = 0; j < 8; j++) {  // values e and e + 2 of four a dword
+            const int e = (j / 2) * 4 + (j & 1);
+            const float f0 = v[k][e] * scale, f1 = v[k][e + 2] * scale;
             const _Float16 h0 = (_Float16)f0, h1 = (_Float16)f1;
             const _Float16 l0 = (_Float16)(f0 - (float)h0), l1 = (_Float16)(f1 - (float)h1);
-            hw[j / 2] = __builtin_bit_cast(uint16_t, h0) | (uint32_t)__builtin_bit_cast(uint16_t, h1) << 16;
-            lw[j / 2] = __builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
-            sum += f0 + f1;
+            hw[j] = __builtin_bit_cast(uint16_t, h0) | (uint32_t)__builtin_bit_cast(uint16_t, h1) << 16;
+            lw[j] = __builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
         }
         sum += __shfl_xor(sum, 1, WAVE);
         if (r >= nr) continue;
         const int c = r / 2;  // the 32-value chunk
-        uint8_t *blk = o + (size_t)(c / 8) * 1024 + (c % 8) * 64 + (r & 1) * 32;
-        ((uint4 *)blk)[0] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
-        ((uint4 *)blk)[1] = make_uint4(hw[4], hw[5], hw[6], hw[7]);
-        ((uint4 *)(blk + 512))[0] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
-        ((uint4 *)(blk + 512))[1] = make_uint4(lw[4], lw[5], lw[6], lw[7]);
+        uint8_t *blk = o + (size_t)(c / 8) * 1024 + hact_piece(c % 8, 2 * (r & 1));
+        *(uint4 *)blk = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+        *(uint4 *)(blk + 64) = make_uint4(lw[0], lw[1], lw[2], lw[3]);
+        *(uint4 *)(blk + 256) = make_uint4(hw[4], hw[5], hw[6], hw[7]);
+        *(uint4 *)(blk + 320) = make_uint4(lw[4], lw[5], lw[6], lw[7]);
         if ((r & 1) == 0) {
             const float xs = sum * (1.0f / 32);
             const _Float16 xh = (_Float16)xs, xl = (_Float16)(xs - (float)xh);

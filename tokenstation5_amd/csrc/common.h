@@ -147,10 +147,15 @@ __host__ __device__ inline size_t mact_bytes(int64_t n) { return align_up((size_
 // multiple of 256): each token's values scaled by a power of two, 2^-e, that
 // puts the largest in [2^13, 2^14), then split into two fp16 planes,
 // x 2^-e = hi + lo to about 22 bits:
-//   per 256-value block: hi[256] f16, lo[256] f16     (1 KB)
-//   then per 64-value quarter of a block, the sums X of its two 32-value
-//   chunks (of x 2^-e, divided by 32) as fp16 hi + lo: (hi_0, hi_1) (lo_0, lo_1)
-//   (8 bytes), then 2^e (f32).
+//   per 256-value block 64 pieces of 8 values (16 bytes, 1 KB in all), in the
+//   order the matmul's stages read them: [eighth e of a sub-block, 0..3][low or
+//   high sub-block of a pair][plane hi, lo][pair 0..3], values 8 e .. 8 e + 7 of
+//   sub-block 2 pair + (0 low, 1 high), each four values stored as 0, 2, 1, 3;
+//   then per sub-block pair the sums X of its two 32-value sub-blocks (of x
+//   2^-e, divided by 32) as fp16 hi + lo: (hi_0, hi_1) (lo_0, lo_1) (8 bytes),
+//   then 2^e (f32).
+// Where the hi piece of values 8 e .. of sub-block sb sits in its block (lo: 64 bytes on).
+__host__ __device__ inline int hact_piece(int sb, int e) { return 256 * e + 128 * (sb & 1) + 16 * (sb >> 1); }
 __host__ __device__ inline size_t hact_x(int64_t n) { return (size_t)(n / 256) * 1024; }
 __host__ __device__ inline size_t hact_unscale(int64_t n) { return hact_x(n) + (size_t)(n / 32) * 4; }
 __host__ __device__ inline size_t hact_bytes(int64_t n) { return align_up(hact_unscale(n) + 4, 256); }

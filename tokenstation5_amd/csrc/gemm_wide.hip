@@ -7,7 +7,7 @@
 // so per 256-value block
 //   y += d * sum_s sum_k (sc_s q_k) x_k  -  dmin * sum_s m_s X_s
 // with X_s the sub-block's sum of x. Both inner sums run on the matrix cores:
-//  * sc_s q <= 945 is an exact fp16 integer, so the A operand carries the
+//  * sc_s q <= 945 is an exact fp16 integer, so the weight operand carries the
 //    sub-block scale and one fp32 accumulator P collects all 8 sub-blocks of a
 //    block (16 v_mfma_f32_16x16x32_f16 per 16x16 tile and block);
 //  * the activations arrive as two fp16 planes of x 2^-e (hi + lo, about 22
@@ -19,22 +19,40 @@
 // Per block and output only y += d P - 32 dmin Q is left for the VALU, and
 // y = acc 2^e at the end.
 //
-// Workgroup: 4 waves x (2 row tiles of 16) x 128 tokens (8 token tiles): GLU
-// waves take 16 rows of gate and the same 16 of up, the others 32 rows. The K
-// loop runs in stages of a quarter block (64 values, two sub-blocks), two
-// stages in LDS: the one computed and the next, brought in by DMA
-// (global_load_lds_*, from an SGPR or per-lane base and fixed per-lane
-// offsets) while the current one is computed. The loop issues no register
-// loads, so the only waits are the explicit vmcnt ones. A token's 16 pieces of
-// 16 bytes per stage sit at piece ^ (token & 15), so the 16 lanes that read
-// one piece of 16 tokens hit 16 different bank groups. Split-K (grid z, whole
-// blocks) when rows x tokens alone give too few workgroups; a second kernel
-// adds the partial sums in a fixed order.
+// Lane layout of the 16x16x32 MFMA: A lane l = token l%16, k-group l/16 (8
+// values); B lane l = weight row l%16, the same k-group; D lane l = tokens
+// 4*(l/16)+i of row l%16 (16x16x16: 4 values per k-group, the same D), so a
+// lane needs only its own row's d and dmin. The k order inside an MFMA only
+// has to agree between A and B: k-group k takes sub-blocks 2k and 2k + 1 of
+// the block, whose 64 quants are 32 consecutive bytes of the row and whose
+// scales are the only ones the lane decodes, once per block. Stage S (of 4)
+// of a block is quant bytes 8 S .. 8 S + 7 of every k-group: low nibbles
+// (sub-block 2k) one MFMA step, high nibbles (2k + 1) the next. The
+// activation records (hact_*) are stored in that order.
 //
-// Lane layout of the 16x16x32 MFMA: A lane l = row l%16, k-group l/16 (8
-// values); B lane l = token l%16, the same k-group; D lane l = rows
-// 4*(l/16)+i of token l%16 (16x16x16: 4 values per k-group, the same D). The
-// k order inside an MFMA only has to agree between A and B.
+// Workgroup: RG waves, each RT row tiles of 16 (GLU: half of gate, half of up)
+// x TT token tiles of 16. LDS holds four stages of activations (32
+// values of every token: TOK x 128 bytes), two blocks of the weight rows (144
+// bytes a row, as stored) and of the tokens' sums, all brought in by DMA
+// (global_load_lds_*) two stages or a block ahead; a wave's DMA source offsets are
+// fixed per lane, and the loop issues no register loads, so the only waits on
+// memory are the explicit vmcnt ones. A token's 8 pieces of 16 bytes per
+// stage sit at piece ^ (token / 2 & 7), so the 16 lanes that read one piece of
+// 16 tokens hit 16 different bank groups; 144-byte rows do so by themselves.
+// Split-K (whole blocks) when rows x tokens alone give too few workgroups; a
+// second kernel adds the partial sums in a fixed order.
+//
+// What bounds it: per 64 values a wave issues 68 MFMAs (1088 cycles of the
+// matrix core, 544 of them also of the vector ALU) and about 95 vector
+// instructions (380 cycles), two waves a SIMD; the loop takes about 1.6 times
+// the matrix core's time, at 2.2 GHz. It was twice that with the pieces read
+// right before their MFMAs. Gate/up of 256 tokens, 14336 x 4096: 152 us before
+// (64 of gate and up a 4-wave workgroup, two a CU, LDS reads and the unpack in
+// front of the MFMAs), 114 us now (527 TFLOP/s of useful products, twice that
+// issued); down 86 -> 57 us, QKV 54 -> 32 us, wo 37 -> 23 us, the last three
+// also by the outputs' way through LDS. 64 weight rows a wave (half the LDS
+// reads) measured slower: four waves of 64 rows x 128 tokens 138 us, eight of 64
+// x 64 151 us (their unpack is made twice, or no second wave hides the waits).
 #include <algorithm>
 
 #include "common.h"
@@ -55,242 +73,449 @@ struct WideArgs {
     const float *y_in;      // W_ADD: residual [M][ldy] (may be out)
     int64_t ldy;
     int nrows, nb, n_in, M, ks;
-    int gelu;  // W_GLU: GELU (tanh form) for SiLU
+    int units, ntt;         // (row tile, split) units; token tiles of each
+    int gelu;               // W_GLU: GELU (tanh form) for SiLU
 };
 
 enum { W_STORE = 0, W_ADD = 1, W_GLU = 2 };
-constexpr int WG_TOK = 128;
-__host__ __device__ constexpr int wide_rows(int mode) { return mode == W_GLU ? 64 : 128; }
 
-// LDS: two stages of 39 KB (two workgroups per CU).
-struct WideStage {
-    uint4 b[WG_TOK * 16];  // [token][piece ^ (token & 15)]: hi pieces 0..7, lo 8..15
-    uint2 x[WG_TOK];       // [token]: (hi_0, hi_1), (lo_0, lo_1) of the quarter's sums / 32
-    uint4 wq[4][32][2];    // [wave][pair * 16 + row]: the 32 quant bytes of sub-blocks 2 q4, 2 q4 + 1
-    uint4 wh[4][32];       // [wave][pair * 16 + row]: block header (d, dmin, scales)
+template <int MODE_, int RT_, int TT_, int RG_>
+struct WideShape {
+    static constexpr int MODE = MODE_, RT = RT_, TT = TT_, RG = RG_, NT = 64 * RG;
+    static constexpr int WROWS = 16 * RT * RG, ROWS = MODE == W_GLU ? WROWS / 2 : WROWS;  // weight rows, output rows
+    static constexpr int TOK = 16 * TT;
+    static constexpr int PB = TOK * 8 / RG, NB = (PB + 63) / 64;        // activation pieces (16 bytes) a wave and stage, DMAs
+    static constexpr int PW = 16 * RT * 9, NWI = (PW + 63) / 64;   // weight pieces a wave and block, DMAs
+    static constexpr int PX = TOK * 2 / RG;                             // sum pieces a wave and block (one DMA)
+    static_assert(TOK * 8 % RG == 0 && PX <= 64 && RT % 2 == 0, "wide matmul shape");
+};
+template <class SH>
+struct WideLds {
+    uint4 b[4][SH::TOK * 8];     // [token][piece ^ (token / 2 & 7)]: hi pieces of the 4 k-groups, then lo
+    uint4 w[2][SH::WROWS * 9];   // [row group][row]: the row's 144-byte block
+    uint4 x[2][SH::TOK * 2];     // [token][k-group]: (hi_0, hi_1), (lo_0, lo_1) of its sub-blocks' sums / 32
+};
+// Over the same space at the end: the tile's outputs, 4 floats between tokens'
+// rows so that the lane groups of an MFMA result hit different banks.
+template <class SH>
+struct WideOut {
+    float y[SH::TOK][SH::WROWS + 4];
+};
+template <class SH>
+union WideSpace {
+    WideLds<SH> in;
+    WideOut<SH> out;
 };
 
 __device__ inline void dma16s(const uint8_t *sbase, uint32_t voff, uint32_t lds_base) {
     asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds_base) : "memory");
 }
-__device__ inline void dma4s(const uint8_t *sbase, uint32_t voff, uint32_t lds_base) {
-    asm volatile("global_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds_base) : "memory");
-}
 
-// Per-lane DMA sources of a workgroup (constant over the K loop but for the
-// block offset).
-struct WideLanes {
-    uint32_t act[8];     // activation pieces 64 (8 wave + i) + lane: token and piece offsets
-    uint32_t xs;         // quarter sums: token 32 wave + lane / 2, dword lane & 1
-    const uint8_t *q;    // quants: (pair, row) = (lane / 32, lane / 2 % 16), half lane & 1 (block 0)
-    const uint8_t *hdr;  // headers: (pair, row) = (lane / 16, lane % 16), lanes < 32 (block 0)
+// A row's block header, as the lane needs it: the scales and mins of its two
+// sub-blocks (bytes sc_0, sc_1, m_0, m_1) and the (d, dmin) halves.
+struct WideHdr {
+    uint32_t sm, dd;
 };
-
-// Stage (block b, quarter Q4) into LDS stage S.
-template <int Q4>
-__device__ inline void wide_issue(const WideArgs &a, WideStage &S, int b, int wave, int lane, const WideLanes &o,
-                                  const uint8_t *act_base) {
-    const uint8_t *ab = act_base + (int64_t)b * 1024 + Q4 * 128;
-#pragma unroll
-    for (int i = 0; i < 8; i++) dma16s(ab, o.act[i], lds_addr(S.b) + 1024 * (8 * wave + i));
-    dma4s(act_base + hact_x(a.n_in) + (int64_t)(4 * b + Q4) * 8, o.xs, lds_addr(&S.x[32 * wave]));
-    dma16(o.q + (int64_t)b * Q4K_BYTES + 32 * Q4, lds_addr(&S.wq[wave][0][0]));
-    if (lane < 32) dma16(o.hdr + (int64_t)b * Q4K_BYTES, lds_addr(&S.wh[wave][0]));
+__device__ inline WideHdr wide_hdr(uint4 h, int kq) {
+    const int s = 16 * (kq & 1);
+    const uint32_t A = h.y >> s, B = h.z >> s, C = h.w >> s;
+    const uint32_t split = 0u - (uint32_t)(kq >> 1);  // sub-blocks 4-7: low 4 bits from C, top 2 from A or B
+    const uint32_t sc = (((C & 0x0F0Fu) | ((A >> 2) & 0x3030u)) & split) | (A & 0x3F3Fu & ~split);
+    const uint32_t m = ((((C >> 4) & 0x0F0Fu) | ((B >> 2) & 0x3030u)) & split) | (B & 0x3F3Fu & ~split);
+    return WideHdr{sc | m << 16, h.x};
+}
+// Bytes `sel` (two) of v as fp16 integers: 0x64bb is 1024 + b.
+__device__ inline v2h bytes_f16(uint32_t v, uint32_t sel) {
+    return __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, v, sel)) - v2h{(_Float16)1024, (_Float16)1024};
 }
 
-// 8 quants (one nibble of each of 8 bytes) times the sub-block scale, as
-// exact fp16 integers (q sc <= 945): byte -> 0x64bb is 1024 + q, and
+// A wave's registers over the K loop.
+template <class SH>
+struct WideRegs {
+    v4f acc[SH::RT][SH::TT];      // tokens 4 kq + i of the lane's row
+    v4f P[SH::RT][SH::TT];        // the block's sum of sc q x
+    v4f Q[SH::RT / 2];            // half the row tiles' sums of m X / 32, of one token tile
+    WideHdr hd[SH::RT], hn[SH::RT];  // the row's header, this block's and the next's
+    uint2 q[SH::RT];              // the lane's 8 quant bytes of a pair of stages
+    v2h sc[SH::RT], off[SH::RT];  // (sc_0, sc_1), (-1024 sc_0, -64 sc_1)
+    v8h W[2][SH::RT];             // the weights of a stage's low and high nibbles
+    v8h f[4];                     // the activations of the next tile steps, a ring
+};
+// The lane's quants of stages 2 S and 2 S + 1 from LDS (`wl`: its first row's block).
+template <class SH>
+__device__ inline void wide_read_q(const uint8_t *wl, WideRegs<SH> &R, int S, int kq) {
+#pragma unroll
+    for (int p = 0; p < SH::RT; p++) R.q[p] = *(const uint2 *)(wl + p * 16 * Q4K_BYTES + 16 + 32 * kq + 8 * S);
+}
+template <class SH>
+__device__ inline void wide_scales(WideRegs<SH> &R, int p) {
+    R.hd[p] = R.hn[p];
+    R.sc[p] = bytes_f16(R.hd[p].sm, 0x04010400u);
+    R.off[p] = R.sc[p] * v2h{(_Float16)-1024, (_Float16)-64};
+}
+// Masks and magics of the nibble unpack, opaque to the compiler so that each
+// stays in a register and `and` and `or` become one instruction.
+struct WideConst {
+    uint32_t mask[2], magic[2];
+};
+__device__ inline WideConst wide_const() {
+    WideConst k;
+    asm("v_mov_b32 %0, 0x000F000F" : "=v"(k.mask[0]));
+    asm("v_mov_b32 %0, 0x00F000F0" : "=v"(k.mask[1]));
+    asm("s_mov_b32 %0, 0x64006400" : "=s"(k.magic[0]));
+    asm("s_mov_b32 %0, 0x54005400" : "=s"(k.magic[1]));
+    return k;
+}
+// Pair u (row tile u / 4, pair u % 4 of its 8 values) of the weights of step c:
+// the low (0) or high (1) nibbles of bytes 0 and 2, 1 and 3, 4 and 6, 5 and 7
+// (the activations' order within 8 values) times the sub-block scale, as exact
+// fp16 integers (q sc <= 945). 0x640q is 1024 + q, 0x54q0 is 64 + q;
 // fma(1024 + q, sc, -1024 sc) rounds once, to the exact q sc.
-__device__ inline v8h nib_f16(uint2 q, int hi, v2h sc, v2h off) {
-    const uint32_t v0 = (hi ? q.x >> 4 : q.x) & 0x0F0F0F0Fu, v1 = (hi ? q.y >> 4 : q.y) & 0x0F0F0F0Fu;
-    auto pair = [&](uint32_t v, uint32_t sel) {
-        return __builtin_elementwise_fma(__builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, v, sel)), sc, off);
+template <class SH>
+__device__ inline void wide_pair(WideRegs<SH> &R, const WideConst &K, int u, int c) {
+    const int p = u / 4, k = u % 4;
+    const uint32_t d = k < 2 ? R.q[p].x : R.q[p].y, v = (k & 1) ? d >> 8 : d;
+    const v2h n = __builtin_bit_cast(v2h, (v & K.mask[c]) | K.magic[c]);
+    const v2h w = __builtin_elementwise_fma(n, v2h{R.sc[p][c], R.sc[p][c]}, v2h{R.off[p][c], R.off[p][c]});
+    R.W[c][p][2 * k] = w[0], R.W[c][p][2 * k + 1] = w[1];
+}
+
+// Stage I = 2 S + c of a block: tile step j = (token tile g, plane) is one
+// piece per lane and RT MFMAs. Pieces are read from LDS 3 steps ahead of their
+// MFMAs, the last ones from the next stage, and the next stage's weights are
+// made beside this one's MFMAs: a 16 x 16 x 32 MFMA holds the matrix core for 16
+// cycles and the vector ALU for 8, so two vector instructions beside each are
+// free and every further one costs its 4 cycles; they are spread evenly, and
+// nothing but the barrier stands between two stages. `bl`: the lane's first
+// piece place in slot 0; `wl`, `wn`: its first row's block in LDS, this block's
+// and the next's; `xl`: the block's sums of its token (first tile).
+template <class SH, int I>
+__device__ __forceinline__ void wide_stage(const uint8_t *wl, const uint8_t *wn, const uint8_t *const (&bl)[2],
+                                           const uint8_t *xl, WideRegs<SH> &R, const WideConst &K, int kq) {
+    constexpr int RT = SH::RT, TT = SH::TT, S = I / 2, c = I % 2, NJ = 2 * TT, NPAIR = 4 * RT;
+    constexpr int F0 = I * NJ;  // the ring's phase (8 NJ steps a block: a multiple of 4)
+    constexpr bool last = I == 7;
+    auto load = [&](int j) {
+        const int slot = (j < NJ ? I : I + 1) & 3, g = j % NJ / 2, pl = j & 1;
+        R.f[(F0 + j) & 3] = *(const v8h *)(bl[pl] + slot * (SH::TOK * 128) + 2048 * g);
     };
-    const v2h p0 = pair(v0, 0x04010400u), p1 = pair(v0, 0x04030402u), p2 = pair(v1, 0x04010400u),
-              p3 = pair(v1, 0x04030402u);
-    return v8h{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
-__device__ inline v2h h2pair(int v) { return v2h{(_Float16)(float)v, (_Float16)(float)v}; }
-
-struct WideAcc {
-    float acc[2][8][4];  // [pair][token tile][row i]
-    v4f P[2][8];         // the block's sum of sc q x
-    v4h xs[8];           // the lane group's quarter sums (hi_0, hi_1, lo_0, lo_1), per token tile
-    v4h amin[2];         // the lane group's mins (m_2k, m_2k+1, m_2k, m_2k+1), per pair
-};
-
-// One quarter block: Q4 static (its sub-blocks, its lane group for the min
-// term, whether it opens or closes the block).
-template <int Q4>
-__device__ inline void wide_stage(const WideStage &S, WideAcc &R, int wave, int kq, int rl) {
-    v2h sc[2][2], off[2][2];
+    float d[RT], dmin[RT];
+    v2h amin[RT];
+    // Block end: acc += d P - 32 dmin Q with Q = sum(m X / 32), for half the row
+    // tiles of one token tile a step: Q half 0 of tile g is made in step (g, pl
+    // 1), half 1 in the step after; each half is finished a step after its Q.
+    auto mins = [&](int g, int half, uint2 x) {
 #pragma unroll
-    for (int p = 0; p < 2; p++) {
-        const uint4 h = S.wh[wave][16 * p + rl];  // the lane's own row
-        int sc0, m0, sc1, m1;
-        kq_scale_min_pair(Q4, h.y, h.z, h.w, sc0, m0, sc1, m1);
-        sc[p][0] = h2pair(sc0), off[p][0] = h2pair(-1024 * sc0);
-        sc[p][1] = h2pair(sc1), off[p][1] = h2pair(-1024 * sc1);
-        if (kq == Q4) {
-            const _Float16 f0 = (_Float16)(float)m0, f1 = (_Float16)(float)m1;
-            R.amin[p] = v4h{f0, f1, f0, f1};
+        for (int i = 0; i < RT / 2; i++) {
+            const v2h m = amin[half * RT / 2 + i];
+            R.Q[i] = __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(v4h, x), v4h{m[0], m[1], m[0], m[1]},
+                                                           v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         }
+    };
+    auto finish = [&](int g, int half) {
+#pragma unroll
+        for (int i = 0; i < RT / 2; i++) {
+            const int p = half * RT / 2 + i;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                R.acc[p][g][e] = fmaf(d[p], R.P[p][g][e], fmaf(-dmin[p], R.Q[i][e], R.acc[p][g][e]));
+        }
+    };
+    uint2 xq[2];
+    uint4 h[RT];
+    if constexpr (last) {
+#pragma unroll
+        for (int p = 0; p < RT; p++)
+            amin[p] = bytes_f16(R.hd[p].sm, 0x04030402u), d[p] = h2f(R.hd[p].dd & 0xffff),
+            dmin[p] = 32.0f * h2f(R.hd[p].dd >> 16);
     }
 #pragma unroll
-    for (int g = 0; g < 8; g++) {
-        const uint2 xv = S.x[16 * g + rl];
-        if (kq == Q4) R.xs[g] = __builtin_bit_cast(v4h, xv);
-    }
-    uint2 q[2];
+    for (int j = 0; j < NJ; j++) {
+        const int g = j / 2, pl = j & 1;
+        load(j + 3);
+        if (j == 0 && I == 6)
 #pragma unroll
-    for (int p = 0; p < 2; p++) q[p] = *(const uint2 *)((const uint8_t *)&S.wq[wave][16 * p + rl][0] + 8 * kq);
+            for (int p = 0; p < RT; p++) h[p] = *(const uint4 *)(wn + p * 16 * Q4K_BYTES);
+        if (last && pl == 0) xq[g & 1] = *(const uint2 *)(xl + 512 * g);
+        if (j == 0 && c == 1) wide_read_q<SH>(last ? wn : wl, R, last ? 0 : S + 1, kq);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int c = 0; c < 2; c++) {
-        v8h A[2];
-#pragma unroll
-        for (int p = 0; p < 2; p++) A[p] = nib_f16(q[p], c, sc[p][c], off[p][c]);
-#pragma unroll
-        for (int g = 0; g < 8; g++) {
-            const int tok = 16 * g + rl;
-            const v8h bh = __builtin_bit_cast(v8h, S.b[16 * tok + ((4 * c + kq) ^ rl)]);
-            const v8h bl = __builtin_bit_cast(v8h, S.b[16 * tok + ((8 + 4 * c + kq) ^ rl)]);
-#pragma unroll
-            for (int p = 0; p < 2; p++) {
-                const v4f c0 = (Q4 == 0 && c == 0) ? v4f{0.f, 0.f, 0.f, 0.f} : R.P[p][g];
-                R.P[p][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[p], bh, c0, 0, 0, 0);
-                R.P[p][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[p], bl, R.P[p][g], 0, 0, 0);
-            }
+        for (int p = 0; p < RT; p++) {
+            const v4f c0 = (I == 0 && pl == 0) ? v4f{0.f, 0.f, 0.f, 0.f} : R.P[p][g];
+            R.P[p][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(R.f[(F0 + j) & 3], R.W[c][p], c0, 0, 0, 0);
         }
-    }
-    if constexpr (Q4 == 3) {  // block end: acc += d P - 32 dmin sum(m X / 32)
+        // The next stage's weights, over all tile steps, or all but the first
+        // two where their quants (and the next block's scales) come first.
+        constexpr int J0 = c == 1 ? 2 : 0, n = NJ - J0;
+        if (last && j < J0)
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
-            float d[4], dmin[4];
+            for (int p = 0; p < RT; p++)
+                if (p * J0 / RT == j) wide_scales<SH>(R, p);
+        if (j >= J0)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const uint32_t hx = S.wh[wave][16 * p + 4 * kq + i].x;
-                d[i] = h2f(hx & 0xffff), dmin[i] = 32.0f * h2f(hx >> 16);
-            }
-#pragma unroll
-            for (int g = 0; g < 8; g++) {
-                const v4f Q = __builtin_amdgcn_mfma_f32_16x16x16f16(R.amin[p], R.xs[g], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    R.acc[p][g][i] = fmaf(d[i], R.P[p][g][i], fmaf(-dmin[i], Q[i], R.acc[p][g][i]));
-            }
+            for (int u = (j - J0) * NPAIR / n; u < (j - J0 + 1) * NPAIR / n; u++) wide_pair<SH>(R, K, u, 1 - c);
+        if (I == 6 && j >= NJ - RT) R.hn[j - (NJ - RT)] = wide_hdr(h[j - (NJ - RT)], kq);  // the next block's headers
+        if (last) {
+            if (j > 1) finish((j - 2) / 2, pl);
+            if (pl == 1) mins(g, 0, xq[g & 1]);
+            else if (g > 0) mins(g - 1, 1, xq[(g - 1) & 1]);
         }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (last) {
+        finish(TT - 1, 0);
+        mins(TT - 1, 1, xq[(TT - 1) & 1]);
+        finish(TT - 1, 1);
     }
 }
 
-template <int MODE>
-__global__ __launch_bounds__(256, 2) void k_gemm_wide(WideArgs a) {
-    constexpr int RT = MODE == W_GLU ? 1 : 2;  // row tiles per matrix and wave
-    constexpr int ROWS = wide_rows(MODE);
-    __shared__ WideStage st[2];
+template <class SH>
+__global__ __launch_bounds__(SH::NT, 2) void k_gemm_wide(WideArgs a) {
+    constexpr int MODE = SH::MODE, RT = SH::RT, TT = SH::TT;
+    constexpr int RTM = MODE == W_GLU ? RT / 2 : RT;  // row tiles per matrix and wave
+    __shared__ WideSpace<SH> space;
+    __shared__ __align__(16) float us[SH::TOK];  // the tokens' 2^e
+    WideLds<SH> &L = space.in;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, kq = lane >> 4, rl = lane & 15;
-    const int t0 = blockIdx.x * WG_TOK, rw = blockIdx.y * ROWS + 16 * RT * wave;
-    const int bps = (a.nb + a.ks - 1) / a.ks, bk0 = blockIdx.z * bps;
+    // Workgroups go to the 8 XCDs in turn: the token tiles of one unit (row
+    // tile, split) follow each other on one XCD, whose L2 then serves the
+    // weights to all but the first.
+    const int id = blockIdx.x, jx = id >> 3;
+    const int unit = (jx / a.ntt) * 8 + (id & 7);
+    if (unit >= a.units) return;
+    const int t0 = (jx % a.ntt) * SH::TOK, row0 = (unit / a.ks) * SH::ROWS, rw = row0 + 16 * RTM * wave, z = unit % a.ks;
+    const int bps = (a.nb + a.ks - 1) / a.ks, bk0 = z * bps;
     const int nblk = max(0, min(a.nb, bk0 + bps) - bk0);
 
-    WideLanes o;
+    uint32_t oact[SH::NB];
 #pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const int u = 64 * (8 * wave + i) + lane, tok = u >> 4, p = (u & 15) ^ (tok & 15);
-        o.act[i] = (uint32_t)((min(t0 + tok, a.M - 1) - t0) * a.act_stride) + (p >> 3) * 512 + (p & 7) * 16;
+    for (int i = 0; i < SH::NB; i++) {
+        const int u = SH::PB * wave + min(64 * i + lane, SH::PB - 1), tok = u >> 3, p = (u & 7) ^ ((tok >> 1) & 7);
+        oact[i] = (uint32_t)((min(t0 + tok, a.M - 1) - t0) * a.act_stride) + p * 16;
     }
-    o.xs = (uint32_t)((min(t0 + 32 * wave + (lane >> 1), a.M - 1) - t0) * a.act_stride) + 4 * (lane & 1);
-    auto row_base = [&](int pair, int row) {  // block 0 of the pair's row (clamped)
-        const int m = MODE == W_GLU ? pair : 0, rt = MODE == W_GLU ? 0 : pair;
-        return (m ? a.w2 : a.w) + (int64_t)min(rw + 16 * rt + row, a.nrows - 1) * a.nb * Q4K_BYTES;
-    };
-    o.q = row_base(lane >> 5, (lane >> 1) & 15) + 16 + 16 * (lane & 1);
-    o.hdr = row_base((lane >> 4) & 1, rl);
+    const int xu = SH::PX * wave + min(lane, SH::PX - 1);
+    const uint32_t ox = (uint32_t)((min(t0 + (xu >> 1), a.M - 1) - t0) * a.act_stride) + 16 * (xu & 1);
+    const uint8_t *wp[SH::NWI];  // weight pieces of block 0: piece u is 16 bytes u % 9 of the wave's row u / 9 (clamped)
+#pragma unroll
+    for (int i = 0; i < SH::NWI; i++) {
+        const int u = min(64 * i + lane, SH::PW - 1), lr = u / 9, p = lr >> 4;
+        const int row = min(rw + 16 * (p % RTM) + (lr & 15), a.nrows - 1);
+        wp[i] = (MODE == W_GLU && p / RTM ? a.w2 : a.w) + (int64_t)row * a.nb * Q4K_BYTES + 16 * (u % 9);
+    }
     const uint8_t *act_base = a.act + (int64_t)t0 * a.act_stride;
+    const uint8_t *x_base = act_base + hact_x(a.n_in);
 
-    WideAcc R;
+    auto issue_b = [&](int b, int I) {  // stage I of block b -> slot I mod 4
+        const uint8_t *ab = act_base + (int64_t)b * 1024 + I * 128;
+        const uint32_t to = lds_addr(&L.b[I & 3][SH::PB * wave]);
 #pragma unroll
-    for (int p = 0; p < 2; p++)
+        for (int i = 0; i < SH::NB; i++)
+            if (64 * (i + 1) <= SH::PB || lane < SH::PB - 64 * i) dma16s(ab, oact[i], to + 1024 * i);
+    };
+    auto issue_w = [&](int b, int buf) {  // block b's weights and sums -> w[buf], x[buf]: NWI + 1 DMAs
+        const uint32_t wb = lds_addr(&L.w[buf][wave * RT * 16 * 9]);
 #pragma unroll
-        for (int g = 0; g < 8; g++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) R.acc[p][g][i] = 0.f;
+        for (int i = 0; i < SH::NWI; i++)
+            if (64 * (i + 1) <= SH::PW || lane < SH::PW - 64 * i) dma16(wp[i] + (int64_t)b * Q4K_BYTES, wb + 1024 * i);
+        if (SH::PX == 64 || lane < SH::PX) dma16s(x_base + (int64_t)b * 32, ox, lds_addr(&L.x[buf][SH::PX * wave]));
+    };
 
-    if (nblk > 0) wide_issue<0>(a, st[0], bk0, wave, lane, o, act_base);
+    WideRegs<SH> R;
+#pragma unroll
+    for (int p = 0; p < RT; p++)
+#pragma unroll
+        for (int g = 0; g < TT; g++) R.acc[p][g] = v4f{0.f, 0.f, 0.f, 0.f};
+
+    const uint8_t *tb = (const uint8_t *)L.b[0] + rl * 128;
+    const uint8_t *const bl[2] = {tb + 16 * (kq ^ (rl >> 1)), tb + 16 * ((4 + kq) ^ (rl >> 1))};
+    const uint8_t *wr[2], *xr[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        wr[i] = (const uint8_t *)&L.w[i][(wave * RT * 16 + rl) * 9];
+        xr[i] = (const uint8_t *)L.x[i] + rl * 32 + 8 * kq;
+    }
+    const WideConst K = wide_const();
+    // At a stage's start every wave waits for its own DMA of the next stage,
+    // issued two stages ago; the barrier then makes all of it visible and
+    // frees the slot of the stage before, into which the stage after next but
+    // one goes. A block's weights and sums are issued in stage 0 of the block
+    // before, behind that stage's activations, and are waited for in stage 3.
+    constexpr int NB = SH::NB, NW = SH::NWI + 1;  // DMAs of a stage, of a block
+    auto sync = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (64 * wave < SH::TOK && 64 * wave + lane < SH::TOK)
+        dma4(act_base + (int64_t)(min(t0 + 64 * wave + lane, a.M - 1) - t0) * a.act_stride + hact_unscale(a.n_in),
+             lds_addr(&us[64 * wave]));
+    if (nblk > 0) {
+        issue_w(bk0, 0);
+        issue_b(bk0, 0);
+        issue_b(bk0, 1);
+        issue_b(bk0, 2);
+        wait_vm_n<2 * NB>();
+        sync();
+#pragma unroll
+        for (int p = 0; p < RT; p++) R.hn[p] = wide_hdr(*(const uint4 *)(wr[0] + p * 16 * Q4K_BYTES), kq);
+        wide_read_q<SH>(wr[0], R, 0, kq);
+#pragma unroll
+        for (int j = 0; j < 3; j++) R.f[j] = *(const v8h *)(bl[j & 1] + 2048 * (j / 2));
+#pragma unroll
+        for (int p = 0; p < RT; p++) wide_scales<SH>(R, p);
+#pragma unroll
+        for (int u = 0; u < 4 * RT; u++) wide_pair<SH>(R, K, u, 0);
+    }
     for (int bi = 0; bi < nblk; bi++) {
-        const int b = bk0 + bi;
-        // Quarter q4 sits in st[q4 & 1]. Each wave waits for its own DMA (the
-        // only one in flight); the barrier then makes every wave's DMA visible
-        // and frees the other buffer, into which the next quarter goes.
-        wait_vm_n<0>();
-        __syncthreads();
-        wide_issue<1>(a, st[1], b, wave, lane, o, act_base);
-        wide_stage<0>(st[0], R, wave, kq, rl);
-        wait_vm_n<0>();
-        __syncthreads();
-        wide_issue<2>(a, st[0], b, wave, lane, o, act_base);
-        wide_stage<1>(st[1], R, wave, kq, rl);
-        wait_vm_n<0>();
-        __syncthreads();
-        wide_issue<3>(a, st[1], b, wave, lane, o, act_base);
-        wide_stage<2>(st[0], R, wave, kq, rl);
-        wait_vm_n<0>();
-        __syncthreads();
-        if (bi + 1 < nblk) wide_issue<0>(a, st[0], b + 1, wave, lane, o, act_base);
-        wide_stage<3>(st[1], R, wave, kq, rl);
+        const int b = bk0 + bi, buf = bi & 1;
+        const bool more = bi + 1 < nblk;
+        const uint8_t *wl = buf ? wr[1] : wr[0], *wn = buf ? wr[0] : wr[1], *xl = buf ? xr[1] : xr[0];
+        wait_vm_n<NB>();
+        sync();
+        issue_b(b, 3);
+        if (more) issue_w(b + 1, buf ^ 1);
+        wide_stage<SH, 0>(wl, wn, bl, xl, R, K, kq);
+        if (more) wait_vm_n<NB + NW>();
+        else wait_vm_n<NB>();
+        sync();
+        issue_b(b, 4);
+        wide_stage<SH, 1>(wl, wn, bl, xl, R, K, kq);
+        if (more) wait_vm_n<NB + NW>();
+        else wait_vm_n<NB>();
+        sync();
+        issue_b(b, 5);
+        wide_stage<SH, 2>(wl, wn, bl, xl, R, K, kq);
+        wait_vm_n<NB>();
+        sync();
+        issue_b(b, 6);
+        wide_stage<SH, 3>(wl, wn, bl, xl, R, K, kq);
+        wait_vm_n<NB>();
+        sync();
+        issue_b(b, 7);
+        wide_stage<SH, 4>(wl, wn, bl, xl, R, K, kq);
+        wait_vm_n<NB>();
+        sync();
+        if (more) issue_b(b + 1, 0);
+        wide_stage<SH, 5>(wl, wn, bl, xl, R, K, kq);
+        if (more) wait_vm_n<NB>();
+        else wait_vm_n<0>();
+        sync();
+        if (more) issue_b(b + 1, 1);
+        wide_stage<SH, 6>(wl, wn, bl, xl, R, K, kq);
+        if (more) wait_vm_n<NB>();
+        sync();
+        if (more) issue_b(b + 1, 2);
+        // The last block's look-ahead reads stale stage and weight bytes and drops them.
+        wide_stage<SH, 7>(wl, wn, bl, xl, R, K, kq);
     }
 
-    // Rows rw + 16 rt + 4 kq + i (pair p = rt, or p = matrix with GLU),
-    // tokens t0 + 16 g + rl.
+    // The outputs to LDS (lane: row rw + 16 rt + rl of matrix m, tokens 16 g + 4
+    // kq + i), then to memory in whole lines: stored straight from the MFMA
+    // layout, 64 bytes a token and instruction, they took 16-20 us of a launch
+    // over 256 tokens.
+    wait_vm_n<0>();
+    __syncthreads();
+    const bool part = a.ks > 1;
+    const int width = MODE == W_GLU && !part ? SH::ROWS : SH::WROWS;  // GLU partials: gate's rows, then up's
 #pragma unroll
-    for (int g = 0; g < 8; g++) {
-        const int tok = t0 + 16 * g + rl;
-        if (tok >= a.M) continue;
-        const float us = *(const float *)(a.act + (int64_t)tok * a.act_stride + hact_unscale(a.n_in));
+    for (int g = 0; g < TT; g++) {
+        const float4 uv = *(const float4 *)&us[16 * g + 4 * kq];
+        const float u4[4] = {uv.x, uv.y, uv.z, uv.w};
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++)
+        for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int r = rw + 16 * rt + 4 * kq + i;
-                if (r >= a.nrows) continue;
-                const float v = R.acc[rt][g][i] * us;
-                if (a.ks > 1) {
-                    float *p = a.out + (((int64_t)blockIdx.z * 2) * a.M + tok) * a.nrows + r;
-                    p[0] = v;
-                    if (MODE == W_GLU) p[(int64_t)a.M * a.nrows] = R.acc[1][g][i] * us;
-                } else {
-                    const int64_t o2 = (int64_t)tok * a.ldy + r;
-                    if (MODE == W_ADD) a.out[o2] = a.y_in[o2] + v;
-                    else if (MODE == W_GLU) a.out[o2] = glu_act(v, R.acc[1][g][i] * us, a.gelu);
-                    else a.out[o2] = v;
-                }
+            for (int rt = 0; rt < RTM; rt++) {
+                float *o = &space.out.y[16 * g + 4 * kq + i][16 * (RTM * wave + rt) + rl];
+                const float v = R.acc[rt][g][i] * u4[i];
+                if constexpr (MODE == W_GLU) {
+                    const float up = R.acc[RTM + rt][g][i] * u4[i];
+                    if (part) o[0] = v, o[SH::ROWS] = up;
+                    else o[0] = glu_act(v, up, a.gelu);
+                } else o[0] = v;
             }
+    }
+    __syncthreads();
+    const int64_t ld = part ? a.nrows : a.ldy;
+    const int64_t plane = (int64_t)a.M * a.nrows;
+    float *out = part ? a.out + 2 * z * plane : a.out;
+    const bool vec = ld % 4 == 0 && (uintptr_t)out % 16 == 0 && plane % 4 == 0 &&
+                     (MODE != W_ADD || part || (uintptr_t)a.y_in % 16 == 0);
+    for (int e = threadIdx.x; e < SH::TOK * width / 4; e += SH::NT) {
+        const int t = e / (width / 4), c = 4 * (e % (width / 4));
+        const int m = MODE == W_GLU && c >= SH::ROWS ? 1 : 0, r = row0 + c - m * SH::ROWS;
+        if (t0 + t >= a.M || r >= a.nrows) continue;
+        float4 v = *(const float4 *)&space.out.y[t][c];
+        const int64_t o = m * plane + (t0 + t) * ld + r;
+        if (vec && r + 4 <= a.nrows) {
+            if (MODE == W_ADD && !part) {
+                const float4 y = *(const float4 *)(a.y_in + o);
+                v.x = y.x + v.x, v.y = y.y + v.y, v.z = y.z + v.z, v.w = y.w + v.w;
+            }
+            *(float4 *)(out + o) = v;
+        } else {
+            const float f[4] = {v.x, v.y, v.z, v.w};
+            for (int i = 0; i < min(4, a.nrows - r); i++)
+                out[o + i] = MODE == W_ADD && !part ? a.y_in[o + i] + f[i] : f[i];
+        }
     }
 }
 
-// Splits of K (whole blocks) that give about two workgroups per CU.
-int wide_splits(int64_t rows, int M, int nb, int cus, int mode) {
-    const int64_t wgs = ((rows + wide_rows(mode) - 1) / wide_rows(mode)) * ((M + WG_TOK - 1) / WG_TOK);
-    const int64_t want = (2 * (int64_t)cus + wgs / 2) / wgs;
-    return (int)std::max<int64_t>(1, std::min<int64_t>({16, want, (int64_t)nb / 2}));
+// The launch of a batch of M tokens: token tiles of at most 128, evened out
+// and rounded up to a built count of 16-token groups (37 tokens in a 48-token
+// tile: the 13824 x 5120 gate/up 42 us, 95 us in a 128-token one); past 48
+// tokens one 8-wave workgroup a CU of 256 weight rows, below it two 4-wave
+// workgroups of 128, whose barriers don't hold each other up (the 14336 x 4096
+// gate/up of 20 tokens 26 against 30 us, of 37 tokens 42 against 44, of 64
+// tokens 41 against 40); splits of K (whole blocks) that fill those slots.
+struct WidePlan {
+    int tt, rows, ntt, ks;
+};
+static WidePlan wide_plan(int64_t rows, int M, int nb, int cus, int mode) {
+    WidePlan p;
+    p.ntt = (M + 127) / 128;
+    const int need = ((M + p.ntt - 1) / p.ntt + 15) / 16;
+    p.tt = need <= 2 ? 2 : need <= 4 ? need : need <= 6 ? 6 : 8;
+    p.ntt = (M + 16 * p.tt - 1) / (16 * p.tt);
+    p.rows = (p.tt > 3 ? 256 : 128) / (mode == W_GLU ? 2 : 1);
+    const int64_t wgs = ((rows + p.rows - 1) / p.rows) * p.ntt, slots = (p.tt > 3 ? 1 : 2) * (int64_t)cus;
+    const int64_t want = (slots + wgs / 2) / wgs;
+    p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({16, want, (int64_t)nb / 2}));
+    return p;
+}
+int wide_splits(int64_t rows, int M, int nb, int cus, int mode) { return wide_plan(rows, M, nb, cus, mode).ks; }
+
+template <int MODE, int TT>
+static hipError_t wide_go(WideArgs &a, const WidePlan &p, hipStream_t s) {
+    using SH = WideShape<MODE, 2, TT, (TT > 3 ? 8 : 4)>;
+    a.units = (a.nrows + SH::ROWS - 1) / SH::ROWS * a.ks, a.ntt = p.ntt;
+    hipLaunchKernelGGL((k_gemm_wide<SH>), dim3((unsigned)(8 * a.ntt * ((a.units + 7) / 8))), dim3(SH::NT), 0, s, a);
+    return hipGetLastError();
+}
+template <int MODE>
+static hipError_t wide_mode(WideArgs &a, const WidePlan &p, hipStream_t s) {
+    switch (p.tt) {
+    case 2: return wide_go<MODE, 2>(a, p, s);
+    case 3: return wide_go<MODE, 3>(a, p, s);
+    case 4: return wide_go<MODE, 4>(a, p, s);
+    case 6: return wide_go<MODE, 6>(a, p, s);
+    default: return wide_go<MODE, 8>(a, p, s);
+    }
 }
 
 hipError_t launch_gemm_wide(const void *w, const void *w2, int64_t ne0, int64_t ne1, const void *act, int M, int mode,
-                            float *y, const float *y_in, int64_t ldy, void *scratch, int ks, hipStream_t s) {
+                            float *y, const float *y_in, int64_t ldy, void *scratch, int cus, hipStream_t s) {
     WideArgs a{};
     a.gelu = (mode & GLU_GELU) ? 1 : 0;
     mode &= ~GLU_GELU;
+    const WidePlan p = wide_plan(ne1, M, (int)(ne0 / 256), cus, mode);
     a.w = (const uint8_t *)w, a.w2 = (const uint8_t *)w2, a.act = (const uint8_t *)act;
     a.act_stride = (int64_t)hact_bytes(ne0), a.y_in = y_in, a.ldy = ldy;
-    a.nrows = (int)ne1, a.nb = (int)(ne0 / 256), a.n_in = (int)ne0, a.M = M, a.ks = ks;
-    a.out = ks > 1 ? (float *)scratch : y;
-    const int rows = wide_rows(mode);
-    const dim3 grid((unsigned)((M + WG_TOK - 1) / WG_TOK), (unsigned)((ne1 + rows - 1) / rows), (unsigned)ks);
-    if (mode == W_GLU) hipLaunchKernelGGL(k_gemm_wide<W_GLU>, grid, dim3(256), 0, s, a);
-    else if (mode == W_ADD) hipLaunchKernelGGL(k_gemm_wide<W_ADD>, grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(k_gemm_wide<W_STORE>, grid, dim3(256), 0, s, a);
-    return hipGetLastError();
+    a.nrows = (int)ne1, a.nb = (int)(ne0 / 256), a.n_in = (int)ne0, a.M = M, a.ks = p.ks;
+    a.out = p.ks > 1 ? (float *)scratch : y;
+    if (mode == W_GLU) return wide_mode<W_GLU>(a, p, s);
+    if (mode == W_ADD) return wide_mode<W_ADD>(a, p, s);
+    return wide_mode<W_STORE>(a, p, s);
 }
 
 }  // namespace ts5hip
