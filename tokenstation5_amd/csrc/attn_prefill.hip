@@ -19,9 +19,11 @@
 //    range), two MFMAs into one fp32 accumulator, then S += ks * R per group.
 //  * online softmax per row in the log2 domain (causal mask, running max m and
 //    sum l; the rows are the lanes' columns, so only 4-lane exchanges).
-//  * O^T (d x rows) += V^T . P^T on v_mfma_f32_16x16x16_f16, whose B operand
-//    layout is exactly the D layout of the S^T tiles: P stays in registers as
-//    fp16 hi + lo; Vh Ph + Vl Ph + Vh Pl.
+//  * O^T (d x rows) += V^T . P^T on v_mfma_f32_16x16x32_f16: the k order only
+//    has to agree between the operands, so a k-group's 8 keys are the 4 of the
+//    lane in each of two S^T tiles (the D layout is the B layout) and P stays in
+//    registers as fp16 hi + lo; Vh Ph + Vl Ph + Vh Pl. V^T is kept in units of
+//    those 8 keys (16 bytes).
 // Several key splits write (m, l, O) partials that a second kernel merges in
 // split order; one split writes O / l directly.
 //
@@ -30,6 +32,17 @@
 // buffers, the next block's while this one is computed), V's raw block is
 // transposed into V^T, S needs no scale and the value product no lo plane of
 // V (Vh Ph + Vh Pl).
+//
+// What bounds it: the vector ALU. Per block of 64 keys a wave issues 160 MFMAs
+// (2560 cycles of the matrix core, half of them also the vector ALU's) and, for
+// q8, about 560 vector instructions (2240 cycles): the scores' scales, the
+// softmax, the split of P and its share of the K and V conversion. So the
+// conversion works in packed fp16 (v8 vs is exact in 19 bits, hi = RN(v8 vs) and
+// lo = v8 vs - hi as packed multiply and fma: 88 instructions where fp32 took
+// 210), the exponent is one fma and one v_exp, the mask a compare against the
+// lane's own limit, and the value product takes 32 keys an MFMA (16 before, at
+// the same 16 cycles). 256 queries over 4096 keys, 32/8 heads of 128: q8 82 ->
+// 58 us, f16 63 -> 50 us (the merge of the key splits, 9.5 us, beside it).
 #include <algorithm>
 
 #include "common.h"
@@ -57,6 +70,11 @@ constexpr int PF_ROWS = 128;  // query rows per workgroup
 // The k16 tiles' swizzle: unit u of key k sits at u ^ (k & pf_ksw(HD)), a
 // permutation of the key's HD / 8 units.
 __host__ __device__ constexpr int pf_ksw(int hd) { return hd / 8 - 1 < 15 ? hd / 8 - 1 : 15; }
+// V^T's swizzle: the 16 rows d of a tile read one unit, and 8 threads 4 rows
+// apart write one, both without bank conflicts. Unit u holds keys pf_vkey(u)
+// .. + 3 and the four 16 on.
+__device__ inline int pf_vsw(int d) { return ((d >> 1) ^ (d >> 4)) & 7; }
+__device__ inline int pf_vkey(int u) { return 32 * (u >> 2) + 4 * (u & 3); }
 constexpr float PF_LOG2E = 1.4426950408889634f;
 
 template <int HD, bool F16>
@@ -70,15 +88,15 @@ struct PfLds<HD, false> {
     uint16_t vs[PF_KB][HD / 32];
     uint4 k16[PF_KB][HD / 8];      // k8 as fp16, unit u of key k at u ^ (k & pf_ksw(HD))
     float ksf[HD / 32][PF_KB];     // K scales, [group][key]
-    uint2 vh[HD][PF_KB / 4];       // V^T hi, key quad q of row d at q ^ (d & 15)
-    uint2 vl[HD][PF_KB / 4];       // V^T lo
+    uint4 vh[HD][PF_KB / 8];       // V^T hi, unit u of row d at u ^ pf_vsw(d)
+    uint4 vl[HD][PF_KB / 8];       // V^T lo
 };
 
 template <int HD>
 struct PfLds<HD, true> {
     uint4 k16[2][PF_KB][HD / 8];  // K as stored (DMA), unit u of key k at u ^ (k & pf_ksw(HD)); two blocks in turn
     uint16_t v16[PF_KB][HD];      // raw V block (DMA)
-    uint2 vh[HD][PF_KB / 4];      // V^T, key quad q of row d at q ^ (d & 15)
+    uint4 vh[HD][PF_KB / 8];      // V^T, unit u of row d at u ^ pf_vsw(d)
 };
 
 // Raw block at key kb (keys past n_ctx read the last slot; they are masked).
@@ -125,29 +143,26 @@ __device__ inline void pf_issue(const PfArgs &a, PfLds<HD, true> &L, int64_t slo
 // Raw V -> V^T (keys at or past kend: V = 0); K is already in place.
 template <int HD>
 __device__ inline void pf_convert(PfLds<HD, true> &L, int kb, int kend) {
-    constexpr int DQ = HD / 4;  // d quads; thread = (4 consecutive d, 8 consecutive keys)
+    constexpr int DQ = HD / 4;  // d quads; thread = (4 consecutive d, a unit of 8 keys)
     for (int w = threadIdx.x; w < DQ * (PF_KB / 8); w += 256) {
-        const int dq = w % DQ, k0 = 8 * (w / DQ), d0 = 4 * dq;
+        const int dq = w % DQ, u = w / DQ, k0 = pf_vkey(u), d0 = 4 * dq;
         uint32_t hw[4][4];  // [d][key pair]
 #pragma unroll
-        for (int kk = 0; kk < 8; kk += 2) {
+        for (int t = 0; t < 4; t++) {
             uint2 r[2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                const int key = k0 + kk + e;
+                const int key = k0 + 16 * (t >> 1) + 2 * (t & 1) + e;
                 r[e] = kb + key < kend ? *(const uint2 *)&L.v16[key][d0] : make_uint2(0u, 0u);
             }
-            hw[0][kk / 2] = (r[0].x & 0xffffu) | (r[1].x << 16);
-            hw[1][kk / 2] = (r[0].x >> 16) | (r[1].x & 0xffff0000u);
-            hw[2][kk / 2] = (r[0].y & 0xffffu) | (r[1].y << 16);
-            hw[3][kk / 2] = (r[0].y >> 16) | (r[1].y & 0xffff0000u);
+            hw[0][t] = (r[0].x & 0xffffu) | (r[1].x << 16);
+            hw[1][t] = (r[0].x >> 16) | (r[1].x & 0xffff0000u);
+            hw[2][t] = (r[0].y & 0xffffu) | (r[1].y << 16);
+            hw[3][t] = (r[0].y >> 16) | (r[1].y & 0xffff0000u);
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int d = d0 + j, q0 = k0 / 4;
-            L.vh[d][q0 ^ (d & 15)] = make_uint2(hw[j][0], hw[j][1]);
-            L.vh[d][(q0 + 1) ^ (d & 15)] = make_uint2(hw[j][2], hw[j][3]);
-        }
+        for (int j = 0; j < 4; j++)
+            L.vh[d0 + j][u ^ pf_vsw(d0 + j)] = make_uint4(hw[j][0], hw[j][1], hw[j][2], hw[j][3]);
     }
 }
 
@@ -179,37 +194,37 @@ __device__ inline void pf_convert(PfLds<HD, false> &L, int kb, int kend) {
         const int key = t / (HD / 32), grp = t % (HD / 32);
         L.ksf[grp][key] = h2f(L.ks[key][grp]);
     }
-    {  // V^T: thread = (4 consecutive d, 8 consecutive keys)
+    {  // V^T: thread = (4 consecutive d, a unit of 8 keys); v8 vs is exact in 19 bits, hi and lo in packed fp16
         constexpr int DQ = HD / 4;  // d quads
         for (int w = t; w < DQ * (PF_KB / 8); w += 256) {
-            const int dq = w % DQ, k0 = 8 * (w / DQ), d0 = 4 * dq;
-            uint32_t hw[4][4], lw[4][4];  // [d][key pair]
+            const int dq = w % DQ, u = w / DQ, k0 = pf_vkey(u), d0 = 4 * dq;
+            uint32_t raw[8];
+            v2h s[4];  // the key pairs' scales
 #pragma unroll
-            for (int kk = 0; kk < 8; kk += 2) {
-                float f[2][4];
-#pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const int key = k0 + kk + e;
-                    const uint32_t raw = *(const uint32_t *)&L.v8[key][d0];
-                    const float s = kb + key < kend ? h2f(L.vs[key][d0 / 32]) : 0.f;
-#pragma unroll
-                    for (int j = 0; j < 4; j++) f[e][j] = (float)(int8_t)(raw >> (8 * j)) * s;
-                }
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const _Float16 h0 = (_Float16)f[0][j], h1 = (_Float16)f[1][j];
-                    const _Float16 l0 = (_Float16)(f[0][j] - (float)h0), l1 = (_Float16)(f[1][j] - (float)h1);
-                    hw[j][kk / 2] = __builtin_bit_cast(uint16_t, h0) | (uint32_t)__builtin_bit_cast(uint16_t, h1) << 16;
-                    lw[j][kk / 2] = __builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
-                }
+            for (int p = 0; p < 4; p++) {
+                const int key = k0 + 16 * (p >> 1) + 2 * (p & 1);
+                raw[2 * p] = *(const uint32_t *)&L.v8[key][d0] ^ 0x80808080u;  // bytes + 128
+                raw[2 * p + 1] = *(const uint32_t *)&L.v8[key + 1][d0] ^ 0x80808080u;
+                const uint32_t s0 = kb + key < kend ? L.vs[key][d0 / 32] : 0u;
+                const uint32_t s1 = kb + key + 1 < kend ? L.vs[key + 1][d0 / 32] : 0u;
+                s[p] = __builtin_bit_cast(v2h, s0 | s1 << 16);
             }
+            const v2h k1152 = {(_Float16)1152.0f, (_Float16)1152.0f};
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const int d = d0 + j, q0 = k0 / 4;
-                L.vh[d][q0 ^ (d & 15)] = make_uint2(hw[j][0], hw[j][1]);
-                L.vh[d][(q0 + 1) ^ (d & 15)] = make_uint2(hw[j][2], hw[j][3]);
-                L.vl[d][q0 ^ (d & 15)] = make_uint2(lw[j][0], lw[j][1]);
-                L.vl[d][(q0 + 1) ^ (d & 15)] = make_uint2(lw[j][2], lw[j][3]);
+                uint32_t hw[4], lw[4];
+#pragma unroll
+                for (int p = 0; p < 4; p++) {
+                    // 0x64xx = 1024 + (v8 + 128), less 1152
+                    const uint32_t b = __builtin_amdgcn_perm(raw[2 * p + 1], raw[2 * p], 0x0c000c00u | (4 + j) << 16 | j);
+                    const v2h v = __builtin_bit_cast(v2h, b | 0x64006400u) - k1152;
+                    const v2h hi = v * s[p];
+                    hw[p] = __builtin_bit_cast(uint32_t, hi);
+                    lw[p] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, s[p], -hi));
+                }
+                const int d = d0 + j, at = u ^ pf_vsw(d);
+                L.vh[d][at] = make_uint4(hw[0], hw[1], hw[2], hw[3]);
+                L.vl[d][at] = make_uint4(lw[0], lw[1], lw[2], lw[3]);
             }
         }
     }
@@ -318,55 +333,59 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(PfArgs a) {
                 }
             }
         }
-        // Online softmax per row (log2 domain).
-        v4h ph[4][2], pl[4][2];
+        __builtin_amdgcn_sched_barrier(0);
+        // Online softmax per row (log2 domain), straight-line (a branch around
+        // the mask or the rescale made the compiler spill 128 registers).
+        v8h ph[2][2], pl[2][2];  // [tile pair][qt]
 #pragma unroll
         for (int qt = 0; qt < 2; qt++) {
+            const int lim = min(pos[qt], kend - 1) - kb - 4 * kq;  // the last key seen, of the lane's 16 kt + i
+#pragma unroll
+            for (int kt = 0; kt < 4; kt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) S[kt][qt][i] = 16 * kt + i > lim ? -INFINITY : S[kt][qt][i];
             float mx = -INFINITY;
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int key = kb + 16 * kt + 4 * kq + i;
-                    const float s = key <= pos[qt] && key < kend ? S[kt][qt][i] * p2e[qt] : -INFINITY;
-                    S[kt][qt][i] = s;
-                    mx = fmaxf(mx, s);
-                }
-            mx = max_xor32(max_xor16(mx));
-            const float mn = fmaxf(m[qt], mx);
-            const float alpha = mn == -INFINITY ? 1.0f : exp2f(m[qt] - mn);
+                for (int i = 0; i < 4; i++) mx = fmaxf(mx, S[kt][qt][i]);
+            mx = max_xor32(max_xor16(mx)) * p2e[qt];
+            const float mn = fmaxf(m[qt], mx), m0 = mn == -INFINITY ? 0.f : mn;  // (no key yet: every p is 0)
+            const float alpha = __builtin_amdgcn_exp2f(m[qt] - m0);
             float sum = 0.f;
 #pragma unroll
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    const float p = mn == -INFINITY ? 0.f : exp2f(S[kt][qt][i] - mn);
+                    const float p = __builtin_amdgcn_exp2f(fmaf(S[kt][qt][i], p2e[qt], -m0));
                     sum += p;
-                    ph[kt][qt][i] = (_Float16)p;
-                    pl[kt][qt][i] = (_Float16)(p - (float)ph[kt][qt][i]);
+                    const _Float16 h = (_Float16)p;
+                    ph[kt / 2][qt][4 * (kt & 1) + i] = h;
+                    pl[kt / 2][qt][4 * (kt & 1) + i] = (_Float16)(p - (float)h);
                 }
             sum = add_xor32(add_xor16(sum));
             m[qt] = mn, l[qt] = l[qt] * alpha + sum;
 #pragma unroll
-            for (int dt = 0; dt < NDT; dt++) O[qt][dt] *= alpha;
+                for (int dt = 0; dt < NDT; dt++) O[qt][dt] *= alpha;
         }
+        __builtin_amdgcn_sched_barrier(0);
         // O^T += V^T P^T.
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++) {
             const int d = 16 * dt + rl;
 #pragma unroll
-            for (int kt = 0; kt < 4; kt++) {
-                const int quad = 4 * kt + kq;
-                const v4h vh = __builtin_bit_cast(v4h, L.vh[d][quad ^ (d & 15)]);
+            for (int k2 = 0; k2 < 2; k2++) {
+                const int at = (4 * k2 + kq) ^ pf_vsw(d);
+                const v8h vh = __builtin_bit_cast(v8h, L.vh[d][at]);
 #pragma unroll
-                for (int qt = 0; qt < 2; qt++) {
-                    O[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(vh, ph[kt][qt], O[qt][dt], 0, 0, 0);
-                    if constexpr (!F16) {
-                        const v4h vl = __builtin_bit_cast(v4h, L.vl[d][quad ^ (d & 15)]);
-                        O[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(vl, ph[kt][qt], O[qt][dt], 0, 0, 0);
-                    }
-                    O[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(vh, pl[kt][qt], O[qt][dt], 0, 0, 0);
+                for (int qt = 0; qt < 2; qt++) O[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, ph[k2][qt], O[qt][dt], 0, 0, 0);
+                if constexpr (!F16) {
+                    const v8h vl = __builtin_bit_cast(v8h, L.vl[d][at]);
+#pragma unroll
+                    for (int qt = 0; qt < 2; qt++) O[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, ph[k2][qt], O[qt][dt], 0, 0, 0);
                 }
+#pragma unroll
+                for (int qt = 0; qt < 2; qt++) O[qt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh, pl[k2][qt], O[qt][dt], 0, 0, 0);
             }
         }
     }
