@@ -486,6 +486,30 @@ def test_attention_merges_every_split(ctx, H, HKV, HD, n, n_split):
     assert rel_l2(out.download(np.float32), want) <= 2e-5
 
 
+@pytest.mark.parametrize("B,H,HKV,p0", [(2, 8, 8, 0), (5, 32, 8, 4096), (16, 16, 8, 3000), (8, 32, 8, 700), (6, 5, 1, 9000)])
+def test_attention_verify_default_splits(ctx, B, H, HKV, p0):
+    """A verify batch's default split count, which the partials of the no-allocation entry point limit
+    (16 queries of 16/8 heads: 24 of 32 splits): both entry points, bit for bit, and the oracle."""
+    HD, n_ctx = 128, p0 + B
+    rng = np.random.default_rng(B * 31 + p0)
+    q8, sc, deq = q8_cache(rng, 1, HKV, n_ctx, HD)
+    v8, vsc, vdeq = q8_cache(rng, 1, HKV, n_ctx, HD)
+    q = rng.standard_normal((B, H * HD)).astype(np.float32)
+    scale = float(np.float32(1) / np.sqrt(np.float32(HD)))
+    args = (ctx.to_device(q), B, H, HKV, HD, ctx.to_device(q8), ctx.to_device(sc), ctx.to_device(v8),
+            ctx.to_device(vsc), n_ctx, ctx.to_device(np.array([p0], np.int32)), 0, scale)
+    got = []
+    for entry in (ctx.attn_decode, ctx.attn_decode_noalloc):
+        out = ctx.alloc(q.nbytes)
+        entry(*args, out)
+        got.append(out.download(np.float32, (B, H * HD)))
+    np.testing.assert_array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+    kc = deq[0].transpose(1, 0, 2).reshape(n_ctx, HKV * HD)
+    vc = vdeq[0].transpose(1, 0, 2).reshape(n_ctx, HKV * HD)
+    for b in range(B):
+        assert rel_l2(got[0][b], oracle.attention(q[b], kc, vc, H, HKV, HD, p0 + b, scale)) <= 2e-5, b
+
+
 def test_attention_most_work_items_twice(ctx):
     """B * HKV = 4096 (the per-op entry point's limit) with 8 key splits each:
     every (query, KV head) merge counter counts 8 workgroups and its last one

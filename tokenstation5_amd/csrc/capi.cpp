@@ -369,7 +369,18 @@ static int attn_decode_into(ts5hip_ctx *ctx, const float *q, int B, int n_head, 
     if (B <= 0 || n_ctx <= 0 || !attn_supported(n_head, n_head_kv, head_dim))
         return fail(ctx, TS5HIP_ERR_UNSUPPORTED, "attention for %d/%d heads of %d", n_head, n_head_kv, head_dim);
     if (B * n_head_kv > 4096) return fail(ctx, TS5HIP_ERR_ARG, "batch of %d x %d KV heads", B, n_head_kv);
-    if (n_split <= 0) n_split = attn_splits(B, n_head_kv, ctx->n_cu);
+    if (n_split <= 0) {
+        n_split = attn_splits(B, n_head_kv, ctx->n_cu);
+        // The multi-query kernel's work items hold all the batch's queries, so
+        // its splits fill the CUs by themselves (5 queries at 4101 keys, 32/8
+        // heads: 6 splits, 48 work items, 29 us; 32 splits 17 us), as many as
+        // the no-allocation scratch holds, so that both entry points agree.
+        if (attn_mq_fits(B, n_head, n_head_kv, head_dim, kv_f16, kv_per_batch)) {
+            const size_t one = attn_partial_bytes(B, 1, n_head, n_head_kv, head_dim);
+            const int fit = (int)((NOALLOC_BYTES - NOALLOC_COUNTER_BYTES) / one);
+            n_split = std::max(n_split, std::min(attn_mq_splits(n_head_kv, ctx->n_cu), fit));
+        }
+    }
     if (n_split > 64) return fail(ctx, TS5HIP_ERR_ARG, "n_split %d (at most 64)", n_split);
     const size_t need = attn_partial_bytes(B, n_split, n_head, n_head_kv, head_dim);
     if (part) {
