@@ -21,6 +21,17 @@
 //   the B layout: P stays in registers; the factor 128 keeps its lo plane
 //   out of the f16 subnormals and leaves O at the end).
 // The waves' (m, l, O) then go through attn_item_out like k_attn's.
+//
+// Up to 4 heads over a q8 cache leave 12 of the 16 columns empty, so column 4 g
+// + h takes head h and scale group g: its query is zero outside the group, so
+// one accumulator holds every group's sums (a lane scales its 4 by its own
+// group's 4 scales, and the groups are added by two row rotations), and its P is
+// scaled by that group's V scales only (O is read from the columns of each
+// dim's own group). Per 16 keys a lane converts 8 scales instead of 32 and
+// splits 4 products into hi + lo instead of 16, about 100 of 330 vector
+// instructions less; these bound the kernel. 16 sequences of 24-32k keys, 32/8
+// heads: 224 -> 210 us (4.8 of the 5.2 TB/s that a copy reaches); a fourth step in
+// flight changes nothing.
 #pragma once
 #include <type_traits>
 
@@ -64,7 +75,9 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
     constexpr float LOG2E = 1.4426950408889634f;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rl = lane & 15, kq = lane >> 4;
-    const bool row_ok = rl < G;  // the lane's column is one of the query's heads
+    constexpr bool GC = !F16 && G <= 4;  // columns (scale group, head)
+    const int head = GC ? rl & 3 : rl, grp = GC ? rl >> 2 : 0;
+    const bool row_ok = head < G;  // the lane's column is one of the query's heads
     const AttnSpan sp = attn_span<16>(a, split, kvh, b, n_split);
     if (split >= sp.used) return;  // an empty split: not counted, not merged
     const int nkeys = max(sp.p1 - sp.p0, 0);
@@ -86,7 +99,8 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
     using Piece = std::conditional_t<F16, u32x4, u32x2>;  // 8 values
     struct Step {
         Piece k[4], v[4];
-        u32x4 ks[F16 ? 1 : 2], vs[F16 ? 1 : 2];
+        u32x4 ks[F16 || GC ? 1 : 2], vs[F16 || GC ? 1 : 2];
+        uint16_t kg[GC ? 4 : 1], vg[GC ? 4 : 1];  // (scale group, head) columns: the lane's group's scales only
     };
     auto piece = [&](__amdgpu_buffer_rsrc_t r, uint32_t e) -> Piece {  // values e .. e + 7
         if constexpr (F16) return __builtin_amdgcn_raw_buffer_load_b128(r, e * 2, 0, 0);
@@ -98,7 +112,14 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
         for (int c = 0; c < 4; c++) w.k[c] = piece(rk, (kl + rl) * HD + 32 * c + 8 * kq);
 #pragma unroll
         for (int i = 0; i < 4; i++) w.v[i] = piece(rv, (kl + 4 * kq + i) * HD + 8 * rl);
-        if constexpr (!F16) {
+        if constexpr (GC) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const uint32_t at = (kl + 4 * kq + i) * 8 + 2 * grp;
+                w.kg[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rks, at, 0, 0);
+                w.vg[i] = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rvs, at, 0, 0);
+            }
+        } else if constexpr (!F16) {
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 w.ks[h] = __builtin_amdgcn_raw_buffer_load_b128(rks, (kl + 4 * kq) * 8 + 16 * h, 0, 0);
@@ -131,7 +152,7 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
     mq_h8 qh[4], ql[4];
     float p2e;
     {
-        const int r = row_ok ? rl : 0;
+        const int r = row_ok ? head : 0;
         float v[4][8], amax = 0.f;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
@@ -149,7 +170,7 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
         for (int c = 0; c < 4; c++)
 #pragma unroll
             for (int j = 0; j < 8; j++) {
-                const float f = v[c][j] * sc;  // exact: sc is a power of 2
+                const float f = !GC || c == grp ? v[c][j] * sc : 0.f;  // exact: sc is a power of 2
                 qh[c][j] = (_Float16)f;
                 ql[c][j] = (_Float16)(f - (float)qh[c][j]);
             }
@@ -164,6 +185,7 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
         const int kl = st * M1_STEP + wave * 16;
         // q8 scales: halfword 4 i + c of the pair of u32x4 is key kl + 4 kq + i, group c.
         float ksf[4][4], vsf[4][4];
+        if constexpr (!GC)
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -174,7 +196,7 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
             }
         // S^T: D[key 4 kq + i][row rl].
         float s[4];
-        if constexpr (F16) {  // one sum over the 128 dims
+        if constexpr (F16 || GC) {  // one sum over the 128 dims (of the column's group)
             mq_f4 R = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -183,7 +205,14 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
                 R = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[c], R, 0, 0, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 4; i++) s[i] = R[i];
+            for (int i = 0; i < 4; i++) {
+                s[i] = R[i];
+                if constexpr (GC) {
+                    s[i] *= h2f(w.kg[i]);
+                    s[i] = dpp_add<0x124, 0xF, true>(s[i]);  // row_ror:4, then 8: the four groups of a head
+                    s[i] = dpp_add<0x128, 0xF, true>(s[i]);
+                }
+            }
         } else {  // a sum per scale group, scaled
 #pragma unroll
             for (int c = 0; c < 4; c++) {
@@ -237,12 +266,15 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
         // x = 128 p * vs rounded to fp32 before its split (the empty asm
         // keeps a contracted product out of the conversions), so that hi + lo
         // is x.
-        mq_h4 ph[4], pl[4];
+        constexpr int NG = GC ? 1 : 4;
+        mq_h4 ph[NG], pl[NG];
 #pragma unroll
-        for (int g = 0; g < 4; g++)
+        for (int g = 0; g < NG; g++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                float x = p[i] * vsf[i][g];
+                float x;
+                if constexpr (GC) x = p[i] * h2f(w.vg[i]);
+                else x = p[i] * vsf[i][g];
                 asm volatile("" : "+v"(x));
                 ph[g][i] = (_Float16)x;
                 pl[g][i] = (_Float16)(x - (float)ph[g][i]);
@@ -253,8 +285,8 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
 #pragma unroll
         for (int dt = 0; dt < 8; dt++) {
             const mq_h4 va = *(const mq_h4 *)&vt[(16 * dt + rl) * MQ_VT + 2 * kq];
-            O[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(va, ph[dt >> 1], O[dt], 0, 0, 0);
-            O[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(va, pl[dt >> 1], O[dt], 0, 0, 0);
+            O[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(va, ph[GC ? 0 : dt >> 1], O[dt], 0, 0, 0);
+            O[dt] = __builtin_amdgcn_mfma_f32_16x16x16f16(va, pl[GC ? 0 : dt >> 1], O[dt], 0, 0, 0);
         }
         // The next step's V^T writes must not pass these reads: in order.
     };
@@ -283,9 +315,10 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
         constexpr float k2m7 = 0.0078125f;  // the factor 128 out (exact)
 #pragma unroll
         for (int dt = 0; dt < 8; dt++)
-            *(float4 *)&S.o_w[wave][rl][16 * dt + 4 * kq] =
-                make_float4(O[dt][0] * k2m7, O[dt][1] * k2m7, O[dt][2] * k2m7, O[dt][3] * k2m7);
-        if (kq == 0) S.m_w[wave][rl] = m, S.l_w[wave][rl] = l;
+            if (!GC || dt >> 1 == grp)
+                *(float4 *)&S.o_w[wave][head][16 * dt + 4 * kq] =
+                    make_float4(O[dt][0] * k2m7, O[dt][1] * k2m7, O[dt][2] * k2m7, O[dt][3] * k2m7);
+        if (kq == 0 && grp == 0) S.m_w[wave][head] = m, S.l_w[wave][head] = l;
     }
     __syncthreads();
     attn_item_out<HD, G, M1_NT>(a, sp, split, kvh, b, n_split, S);
