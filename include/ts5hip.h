@@ -344,7 +344,7 @@ void ts5hip_engine_free(ts5hip_engine *e);
  * its token ids must be the target's. */
 int ts5hip_engine_set_drafter(ts5hip_engine *e, ts5hip_model *dm);
 /* Engine::generate (engine/src/engine.cpp:149-292) with the tokens as ids instead of text:
- * the prompt in 256-token chunks after the prefix already cached, then per step the next token
+ * the prompt in 512-token chunks after the prefix already cached, then per step the next token
  * and up to `draft` drafts (prompt lookup, engine.cpp:134-147, else the draft model,
  * engine.cpp:75-129) forwarded as one batch, each draft kept while the sample at its position
  * equals it. eog: n_eog end-of-generation ids. out: the generated ids (at most max_tokens);

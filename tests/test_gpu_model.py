@@ -207,6 +207,23 @@ def test_long_prompt_logits_and_greedy_match_oracle(ctx, name):
             break
 
 
+def test_prompt_chunks_split_at_512_and_256(ctx):
+    """Prompts go 512 tokens a pass, then 256, then the rest: one 1100-token call (512 + 512 + 76) against
+    the same tokens in calls of 700 (512 + 188) and 400 (256 + 144), and both against the oracle's last row.
+    The two GPU runs' sums run in other orders and can land q8 keys a step apart: the rows are held to the
+    bar of the prompt test above, against the oracle."""
+    hp, tensors, m = load(ctx, "tiny_llama_c", 1200)
+    ref = oracle.Model(hp, tensors, 1200, 2)
+    toks = np.array([(7 + 13 * i + (i * i) % 17) % hp["n_vocab"] for i in range(1100)], np.int32)
+    one = m.forward(toks, 0)[0]
+    m.forward(toks[:700], 0, logits=False)
+    two = m.forward(toks[700:], 700)[0]
+    want = ref.forward(toks, 0)[0]
+    for got in (one, two):
+        err, cos = row_errors(got[None], want[None])
+        assert err.max() <= 2e-3 and cos.min() > 0.999, (err.max(), cos.min())
+
+
 def test_small_batches_wide_ffn_match_oracle(ctx):
     """Batches of 5, 3 and 1 tokens (the verify step's shapes) on a model whose
     ffn is wider than the fused matmul's LDS input (4608 > 4096): the gate/up

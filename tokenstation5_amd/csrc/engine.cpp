@@ -32,9 +32,11 @@ using namespace ts5hip;
 
 namespace {
 
-// Batches of prompt (and draft catch-up) tokens per forward: the reference's
+// Batches of draft catch-up tokens per forward: the reference's
 // chunk (engine.cpp:172, :97), which is also the backend's logits capacity.
 constexpr int kChunk = 256;
+// A prompt goes to the target in the backend's own passes of 512 tokens.
+constexpr int kPromptChunk = 512;
 
 // ---------------------------------------------------------------------------
 // Prompt lookup: a match finder over the history. Every 2-gram (h[j-1], h[j])
@@ -262,8 +264,8 @@ int ts5hip_engine_generate(ts5hip_engine *e, const int32_t *prompt, int n_prompt
     const size_t keep = std::min(common, (size_t)n_prompt - 1);
     h.resize(keep);
     e->drafter.synced = std::min(e->drafter.synced, keep);
-    for (size_t at = keep; at < (size_t)n_prompt; at += kChunk) {
-        const int n = (int)std::min<size_t>(kChunk, (size_t)n_prompt - at);
+    for (size_t at = keep; at < (size_t)n_prompt; at += kPromptChunk) {
+        const int n = (int)std::min<size_t>(kPromptChunk, (size_t)n_prompt - at);
         const bool last = at + (size_t)n == (size_t)n_prompt;
         const int rc = last ? ts5hip_forward_in_place(m, prompt + at, n, (int)at, 0)
                             : ts5hip_forward(m, prompt + at, n, (int)at, nullptr, 0);

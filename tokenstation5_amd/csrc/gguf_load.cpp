@@ -280,7 +280,7 @@ bool hparams_of(const GgufFile &g, ts5hip_hparams &hp, int &n_ctx_train, std::st
 }
 
 // Bytes the model takes in HBM besides its KV cache: the weights in their HBM
-// layouts, the single-token buffers, and the 256-token batch buffers with the
+// layouts, the single-token buffers, and the 512-token batch buffers with the
 // logits rows.
 uint64_t fixed_bytes(const GgufFile &g, const ts5hip_hparams &hp) {
     uint64_t w = 0;
@@ -289,7 +289,7 @@ uint64_t fixed_bytes(const GgufFile &g, const ts5hip_hparams &hp) {
         const size_t db = device_bytes(t.type, t.ne[0], rows);
         w += db ? db : (uint64_t)t.ne[0] * rows * 4;
     }
-    const uint64_t T = 256, E = hp.n_embd, F = hp.n_ff, QR = (uint64_t)(hp.n_head + 2 * hp.n_head_kv) * hp.head_dim;
+    const uint64_t T = 512, E = hp.n_embd, F = hp.n_ff, QR = (uint64_t)(hp.n_head + 2 * hp.n_head_kv) * hp.head_dim;
     const uint64_t act = 4 * T * (2 * E + QR + 2ull * hp.n_head * hp.head_dim + F) + 2 * 4 * T * hp.n_vocab;
     return w + act + (256ull << 20);  // plus scratch: matmul partials, attention partials, top-k
 }
