@@ -467,7 +467,11 @@ __global__ __launch_bounds__(SH::NT, 2) void k_gemm_wide(WideArgs a) {
 // tokens one 8-wave workgroup a CU of 256 weight rows, below it two 4-wave
 // workgroups of 128, whose barriers don't hold each other up (the 14336 x 4096
 // gate/up of 20 tokens 26 against 30 us, of 37 tokens 42 against 44, of 64
-// tokens 41 against 40); splits of K (whole blocks) that fill those slots.
+// tokens 41 against 40); as many splits of K (whole blocks, none empty) as
+// those slots hold at once: rounded to the nearest count, the workgroups past
+// the slots ran a second round (the 11008 x 4096 feed-forward block of 96 tokens 120
+// us, 98 now; the 2816-wide one of 256 tokens 183, 150; the 8B's QKV of 512
+// tokens as 288 workgroups on 256 CUs, its 512-token turn 20.4 ms, 19.8 now).
 struct WidePlan {
     int tt, rows, ntt, ks;
 };
@@ -479,8 +483,9 @@ static WidePlan wide_plan(int64_t rows, int M, int nb, int cus, int mode) {
     p.ntt = (M + 16 * p.tt - 1) / (16 * p.tt);
     p.rows = (p.tt > 3 ? 256 : 128) / (mode == W_GLU ? 2 : 1);
     const int64_t wgs = ((rows + p.rows - 1) / p.rows) * p.ntt, slots = (p.tt > 3 ? 1 : 2) * (int64_t)cus;
-    const int64_t want = (slots + wgs / 2) / wgs;
-    p.ks = (int)std::max<int64_t>(1, std::min<int64_t>({16, want, (int64_t)nb / 2}));
+    const int ks = (int)std::max<int64_t>(1, std::min<int64_t>({16, slots / wgs, (int64_t)nb / 2}));
+    const int per = std::max(1, (nb + ks - 1) / ks);
+    p.ks = std::max(1, (nb + per - 1) / per);  // no split without blocks
     return p;
 }
 int wide_splits(int64_t rows, int M, int nb, int cus, int mode) { return wide_plan(rows, M, nb, cus, mode).ks; }
