@@ -682,6 +682,31 @@ def test_attention_prompt_f16_vs_oracle(ctx, nq, p0, n_ctx, H, HKV, HD):
         assert rel_l2(got[t], want) <= 2e-5, (t, rel_l2(got[t], want))
 
 
+@pytest.mark.parametrize("nq,keys,H", [(256, 4096, 40), (250, 3000, 40), (160, 5000, 40), (200, 4096, 32), (25, 600, 40)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_attention_prompt_split_counts(ctx, nq, keys, H, f16):
+    """Query blocks x 8 KV heads that do not divide 512: 88, 80 and 56 workgroups a split take fewer, longer
+    splits, 56 (32 heads) a short last one past the first round, 8 the most splits that 256 keys each allow."""
+    HKV, HD, p0 = 8, 128, keys - nq
+    rng = np.random.default_rng(nq + keys + H)
+    q = (rng.standard_normal((nq, H * HD)) * 3).astype(np.float32)
+    scale = float(np.float32(1) / np.sqrt(np.float32(HD)))
+    out = ctx.alloc(q.nbytes)
+    if f16:
+        k, v = (rng.standard_normal((1, HKV, keys, HD), dtype=np.float32).astype(np.float16) for _ in range(2))
+        ctx.attn_prompt_f16(ctx.to_device(q), nq, H, HKV, HD, ctx.to_device(k), ctx.to_device(v), keys, p0, scale, out)
+        deq, vdeq = k.astype(np.float32), v.astype(np.float32)
+    else:
+        q8, sc, deq = q8_cache(rng, 1, HKV, keys, HD)
+        v8, vsc, vdeq = q8_cache(rng, 1, HKV, keys, HD)
+        ctx.attn_prompt(ctx.to_device(q), nq, H, HKV, HD, ctx.to_device(q8), ctx.to_device(sc), ctx.to_device(v8),
+                        ctx.to_device(vsc), keys, p0, scale, out)
+    got = out.download(np.float32, (nq, H * HD))
+    kc, vc = (x[0].transpose(1, 0, 2).reshape(keys, HKV * HD) for x in (deq, vdeq))
+    for t in sorted({0, 1, nq // 2, nq - 2, nq - 1}):
+        assert rel_l2(got[t], oracle.attention(q[t], kc, vc, H, HKV, HD, p0 + t, scale)) <= 2e-5, t
+
+
 def test_attention_prompt_large_values_and_bad_shapes(ctx):
     """Queries of 1e6 (past fp16: each row is scaled by a power of two first), keys of
     1e3; then shapes the path does not take are refused, not guessed."""

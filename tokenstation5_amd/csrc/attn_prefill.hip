@@ -454,12 +454,24 @@ bool attn_prefill_supported(int H, int HKV, int HD) {
 }
 
 // Keys per split: a multiple of 64, at least 256, at most 16 splits, and
-// no more splits than bring the launch to about 512 workgroups (wg: the
-// workgroups of one split); every split adds (m, l, O) partials to merge.
+// no more splits than bring the launch to about 512 workgroups, two a CU (wg:
+// the workgroups of one split); every split adds (m, l, O) partials to merge.
+// Workgroups past 512 wait for a second round: fewer, longer splits where one
+// round of them is shorter than two, a short last split in the second.
+// 40/8 heads of 128: 256 queries over 4096 keys as 528 workgroups of 704 keys
+// 112 us (q8) and 82 us (f16), as 440 of 832 keys 88 and 67; 160 over 5000 keys 88
+// -> 67 us. 200 queries of 32/8 heads keep their 56 short ones in a second round
+// (f16, 4096 keys: 47.2 us, 48.4 in one round of 512 keys).
 static int pf_split_keys(int64_t max_keys, int64_t wg) {
     const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(16, (512 + wg - 1) / wg));
-    const int64_t per = std::max<int64_t>(256, (max_keys + splits - 1) / splits);
-    return (int)((per + PF_KB - 1) / PF_KB * PF_KB);
+    const int64_t want = std::max<int64_t>(256, (max_keys + splits - 1) / splits);
+    int64_t best = (want + PF_KB - 1) / PF_KB * PF_KB, least = INT64_MAX;
+    for (int64_t per = best, end = 2 * best; per <= end; per += PF_KB) {
+        const int64_t n = (max_keys + per - 1) / per;
+        const int64_t keys = per + (wg * n <= 512 ? 0 : wg * (n - 1) <= 512 ? max_keys - (n - 1) * per : per);
+        if (keys < least) least = keys, best = per;
+    }
+    return (int)best;
 }
 
 // A bound for every launch with at most max_keys keys (splits <= 16 and
