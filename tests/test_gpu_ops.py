@@ -443,6 +443,30 @@ def test_attention_matrix_core_one_query(ctx, kv, H, HKV):
         assert rel_l2(got[b], want) <= 2e-5, (b, rel_l2(got[b], want))
 
 
+@pytest.mark.parametrize("H,HKV,n_split", [(8, 8, 0), (16, 8, 7), (24, 6, 3), (32, 8, 0), (40, 8, 0)])
+def test_attention_one_query_weights_same_in_every_dim(ctx, H, HKV, n_split):
+    """Every dim of a head is the same weighted mean of V: with V the same in all 128 dims of a key, all
+    128 outputs of a head are the same bits. Keys are one row with a few values a step off, so that scores near
+    1e3 have many near-equal maxima, in every wave and split: a score that one scale group's dims saw an ulp
+    off would show."""
+    HD, n, B = 128, 1500, 2
+    rng = np.random.default_rng(H + 10 * n_split)
+    base = rng.integers(-126, 127, (B, HKV, 1, HD))
+    k8 = (base + rng.integers(-1, 2, (B, HKV, n, HD)) * (rng.random((B, HKV, n, HD)) < 0.05)).astype(np.int8)
+    ks = np.float16(0.13) * (1 + np.arange(4, dtype=np.float16) / 16) * np.ones((B, HKV, n, 4), np.float16)
+    v8 = np.repeat(rng.integers(-127, 128, (B, HKV, n, 1)), HD, -1).astype(np.int8)
+    vs = np.repeat(rng.uniform(0.005, 0.02, (B, HKV, n, 1)).astype(np.float16), 4, -1)
+    q = (rng.standard_normal((B, H * HD)) * 60).astype(np.float32)
+    out = ctx.alloc(q.nbytes)
+    ctx.attn_decode(ctx.to_device(q), B, H, HKV, HD, ctx.to_device(k8), ctx.to_device(ks), ctx.to_device(v8),
+                    ctx.to_device(vs), n, ctx.to_device(np.array([n, n - 41], np.int32)), 1,
+                    float(np.float32(1) / np.sqrt(np.float32(HD))), out, n_split=n_split)
+    got = out.download(np.float32, (B * H, HD))
+    v = v8[..., 0] * vs[..., 0].astype(np.float32)
+    assert np.isfinite(got).all() and np.abs(got).max() <= np.abs(v).max()
+    np.testing.assert_array_equal(got.view(np.uint32), np.repeat(got[:, :1], HD, 1).view(np.uint32))
+
+
 @pytest.mark.parametrize("B,ctxlen,H,HKV,HD,n_split", [(1, 8192, 32, 8, 128, 0), (4, 8192, 32, 8, 128, 0),
                                                        (16, 8192, 32, 8, 128, 0), (1, 32768, 32, 8, 128, 0),
                                                        (4, 32768, 32, 8, 128, 0), (16, 32768, 32, 8, 128, 0),

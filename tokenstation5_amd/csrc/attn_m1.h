@@ -25,12 +25,17 @@
 // Up to 4 heads over a q8 cache leave 12 of the 16 columns empty, so column 4 g
 // + h takes head h and scale group g: its query is zero outside the group, so
 // one accumulator holds every group's sums (a lane scales its 4 by its own
-// group's 4 scales, and the groups are added by two row rotations), and its P is
-// scaled by that group's V scales only (O is read from the columns of each
-// dim's own group). Per 16 keys a lane converts 8 scales instead of 32 and
+// group's 4 scales, and the groups are added by row rotations), and its P is
+// scaled by that group's V scales only. O is read from the columns of each
+// dim's own group and normalised by group 0's m and l, so the four columns of a
+// head must hold the same bits of s: all of them add k0 R0 + k2 R2 and k1 R1 +
+// k3 R3, the first of each fused. Added from each column's own group on, the
+// dims of two groups were weighted by scores an ulp from those behind m and l:
+// 16 sequences of 16384 keys 3.63e-7 from float64, 3.51e-7 now, as with one
+// column a head. Per 16 keys a lane converts 8 scales instead of 32 and
 // splits 4 products into hi + lo instead of 16, about 100 of 330 vector
 // instructions less; these bound the kernel. 16 sequences of 24-32k keys, 32/8
-// heads: 224 -> 210 us (4.8 of the 5.2 TB/s that a copy reaches); a fourth step in
+// heads: 224 -> 211 us (4.8 of the 5.2 TB/s that a copy reaches); a fourth step in
 // flight changes nothing.
 #pragma once
 #include <type_traits>
@@ -208,9 +213,12 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
             for (int i = 0; i < 4; i++) {
                 s[i] = R[i];
                 if constexpr (GC) {
-                    s[i] *= h2f(w.kg[i]);
-                    s[i] = dpp_add<0x124, 0xF, true>(s[i]);  // row_ror:4, then 8: the four groups of a head
-                    s[i] = dpp_add<0x128, 0xF, true>(s[i]);
+                    const float k = h2f(w.kg[i]);
+                    float x = R[i] * k;
+                    asm volatile("" : "+v"(x));
+                    x = fmaf(R[i], k, dpp_mov<0x128, 0xF>(x, x));  // row_ror:8: groups 0 + 2, 1 + 3,
+                    x = dpp_mov<0x128, 0xC>(x, x);                 // in columns 2 and 3 too
+                    s[i] = dpp_add<0x124, 0xF, true>(x);           // row_ror:4
                 }
             }
         } else {  // a sum per scale group, scaled

@@ -255,6 +255,11 @@ template <int CTRL, int ROW_MASK, bool BOUND>
 __device__ inline float dpp_add(float x) {
     return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, ROW_MASK, 0xF, BOUND));
 }
+// x moved by the DPP control, in the 4-lane banks of BANK_MASK; the others keep old.
+template <int CTRL, int BANK_MASK>
+__device__ inline float dpp_mov(float old, float x) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(x), CTRL, 0xF, BANK_MASK, false));
+}
 __device__ inline float wave_sum_dpp(float v) {
     v = dpp_add<0xB1, 0xF, true>(v);    // quad_perm [1,0,3,2]
     v = dpp_add<0x4E, 0xF, true>(v);    // quad_perm [2,3,0,1]
