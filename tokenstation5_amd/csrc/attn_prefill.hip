@@ -349,7 +349,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(PfArgs a) {
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, S[kt][qt][i]);
-            mx = fmaf(max_xor32(max_xor16(mx)), p2e[qt], -7.f);
+            mx = max_xor32(max_xor16(mx)) * p2e[qt];
             const float mn = fmaxf(m[qt], mx), m0 = mn == -INFINITY ? 0.f : mn;  // (no key yet: every p is 0)
             const float alpha = __builtin_amdgcn_exp2f(m[qt] - m0);
             float sum = 0.f;
