@@ -731,6 +731,45 @@ def test_attention_prompt_split_counts(ctx, nq, keys, H, f16):
         assert rel_l2(got[t], oracle.attention(q[t], kc, vc, H, HKV, HD, p0 + t, scale)) <= 2e-5, t
 
 
+@pytest.mark.parametrize("f16", [False, True])
+@pytest.mark.parametrize("HD,below", [(128, 9.5), (128, 12.7), (64, 12.7), (128, 14.6)])
+def test_attention_prompt_weights_far_below_a_sink(ctx, HD, below, f16):
+    """A first key without a value takes 2^below times the weight of every other key (an attention sink), whose
+    values are alike: their weights, not only the largest, need their bits. A weight p is kept as fp16 hi + lo
+    of 128 p, to 2^-25 of 1 at the worst, the other keys' rounding the same way: 2^(below - 31), and 1e-6 for the
+    32-bit sums over 700 keys."""
+    H, HKV, nq, keys = 8, 2, 40, 700
+    q = np.ones((nq, H * HD), np.float32)
+    k = np.zeros((1, HKV, keys, HD), np.float32)
+    k[:, :, 0, :32] = below / 32  # the first key's log2 score; the others' is 0
+    v = np.ones((1, HKV, keys, HD), np.float32)
+    v[:, :, 0] = 0
+    scale = float(np.float32(1) / np.float32(1.4426950408889634))
+    out = ctx.alloc(q.nbytes)
+    if f16:
+        k, v = k.astype(np.float16), v.astype(np.float16)
+        ctx.attn_prompt_f16(ctx.to_device(q), nq, H, HKV, HD, ctx.to_device(k), ctx.to_device(v), keys, keys - nq, scale, out)
+        kd, vd = k.astype(np.float64), v.astype(np.float64)
+    else:
+        def blocks(x):
+            b = x.reshape(1, HKV, keys, HD // 32, 32)
+            s = (np.abs(b).max(-1) / np.float32(127)).astype(np.float16)
+            n = np.rint(b / np.maximum(s.astype(np.float32), 1e-8)[..., None]).clip(-127, 127).astype(np.int8)
+            return n.reshape(x.shape), s, (n * s.astype(np.float64)[..., None]).reshape(x.shape)
+        (k8, ks, kd), (v8, vs, vd) = blocks(k), blocks(v)
+        ctx.attn_prompt(ctx.to_device(q), nq, H, HKV, HD, ctx.to_device(k8), ctx.to_device(ks), ctx.to_device(v8),
+                        ctx.to_device(vs), keys, keys - nq, scale, out)
+    got = out.download(np.float32, (nq, H, HD)).astype(np.float64)
+    for t in (0, nq // 2, nq - 1):
+        n = keys - nq + t + 1
+        for h in range(H):
+            s = kd[0, h // (H // HKV), :n].sum(-1) * scale
+            w = np.exp(s - s.max())
+            want = w @ vd[0, h // (H // HKV), :n] / w.sum()
+            err = np.abs(got[t, h] / want - 1).max()
+            assert err <= 1e-6 + 2.0 ** (below - 31), (t, h, err)
+
+
 def test_attention_prompt_large_values_and_bad_shapes(ctx):
     """Queries of 1e6 (past fp16: each row is scaled by a power of two first), keys of
     1e3; then shapes the path does not take are refused, not guessed."""

@@ -43,6 +43,13 @@
 // lane's own limit, and the value product takes 32 keys an MFMA (16 before, at
 // the same 16 cycles). 256 queries over 4096 keys, 32/8 heads of 128: q8 82 ->
 // 58 us, f16 63 -> 50 us (the merge of the key splits, 9.5 us, beside it).
+//
+// The softmax's reference is the running maximum less 7, so that p goes to 128
+// and l and O carry the factor: a weight's lo plane leaves the fp16 subnormals
+// down to 2^-10 of the largest, not 2^-3 (700 keys with 2^-14.6 of the weight of
+// one without a value: 9.7e-5 from float64 before, 8e-6 at most now; 256 queries of normal
+// scores over 4096 keys 3.40e-7, 3.25e-7 now). Not more than 7: the reference is
+// rounded, and where its last place is 16, less 8 could become less 16 and p 2^16.
 #include <algorithm>
 
 #include "common.h"
@@ -349,7 +356,7 @@ __global__ __launch_bounds__(256, 2) void k_attn_pf(PfArgs a) {
             for (int kt = 0; kt < 4; kt++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, S[kt][qt][i]);
-            mx = max_xor32(max_xor16(mx)) * p2e[qt];
+            mx = fmaf(max_xor32(max_xor16(mx)), p2e[qt], -7.f);  // p to 128: see above
             const float mn = fmaxf(m[qt], mx), m0 = mn == -INFINITY ? 0.f : mn;  // (no key yet: every p is 0)
             const float alpha = __builtin_amdgcn_exp2f(m[qt] - m0);
             float sum = 0.f;
@@ -461,7 +468,10 @@ bool attn_prefill_supported(int H, int HKV, int HD) {
 // 40/8 heads of 128: 256 queries over 4096 keys as 528 workgroups of 704 keys
 // 112 us (q8) and 82 us (f16), as 440 of 832 keys 88 and 67; 160 over 5000 keys 88
 // -> 67 us. 200 queries of 32/8 heads keep their 56 short ones in a second round
-// (f16, 4096 keys: 47.2 us, 48.4 in one round of 512 keys).
+// (f16, 4096 keys: 47.2 us, 48.4 in one round of 512 keys). Longer splits are also
+// longer fp32 sums: 832 keys for 704 took the q8 case from 3.72e-7 to 3.94e-7
+// from float64 (p's factor of 128 took it to 3.76e-7), 512 queries over 2560 keys
+// as 896 for 640 from 3.56e-7 to 3.92e-7 (3.73e-7).
 static int pf_split_keys(int64_t max_keys, int64_t wg) {
     const int64_t splits = std::max<int64_t>(1, std::min<int64_t>(16, (512 + wg - 1) / wg));
     const int64_t want = std::max<int64_t>(256, (max_keys + splits - 1) / splits);
