@@ -2,6 +2,7 @@
 include/ts5hip.h declares, reports layouts and errors without a GPU, and its
 host-side sampler draws exactly as ts5's Engine::sample (engine/src/engine.cpp:16-46).
 No GPU compute runs here."""
+import ctypes
 import os
 import subprocess
 
@@ -97,3 +98,28 @@ def test_synth_layouts_are_whole_blocks():
     # rows (14336 for down) and the Q6_K head over a 128256-token vocabulary.
     wb = synth.weight_bytes(synth.LLAMA_8B)
     assert wb["layers"] == 3925868544 and wb["head"] == 430940160
+
+
+def test_prompt_matmul_splits_fit_every_xcd():
+    """The prompt matmul's splits of K (wide_splits) run in one round: a unit (row tile, split) and its token
+    tiles go to one of the 8 XCDs, units in turn, and an XCD holds 32 of a tile's 8-wave workgroups at a time (64 of the
+    4-wave ones that up to 48 tokens take). No split is empty, and one split is always allowed."""
+    wide_splits = ts5hip.lib()._ZN6ts5hip11wide_splitsEliiii
+    wide_splits.argtypes, wide_splits.restype = [ctypes.c_int64] + [ctypes.c_int] * 4, ctypes.c_int
+    many = 0
+    for glu in (0, 1):
+        for nb in (1, 2, 3, 7, 10, 12, 16, 20, 32, 54, 56):
+            for rows in list(range(128, 8192, 384)) + [896, 3072, 7168, 14336, 33000]:
+                for M in (17, 32, 33, 48, 49, 64, 65, 96, 97, 128, 129, 192, 256, 257, 300, 384, 385, 512, 640, 1024):
+                    ntt = -(-M // 128)
+                    groups = -(-M // ntt)
+                    tt = next(t for t in (2, 3, 4, 6, 8) if 16 * t >= groups)
+                    ntt = -(-M // (16 * tt))
+                    tile = (256 if tt > 3 else 128) // (2 if glu else 1)
+                    ks = wide_splits(rows, M, nb, 256, 2 if glu else 1)
+                    assert 1 <= ks <= max(1, nb // 2) and ks <= 16, (glu, nb, rows, M, ks)
+                    assert (ks - 1) * -(-nb // ks) < nb, (glu, nb, rows, M, ks)
+                    units = -(-rows // tile) * ks
+                    many += ks > 1
+                    assert ks == 1 or -(-units // 8) * ntt <= (32 if tt > 3 else 64), (glu, nb, rows, M, ks)
+    assert many > 1000

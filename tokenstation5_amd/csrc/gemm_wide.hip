@@ -472,6 +472,9 @@ __global__ __launch_bounds__(SH::NT, 2) void k_gemm_wide(WideArgs a) {
 // the slots ran a second round (the 11008 x 4096 feed-forward block of 96 tokens 120
 // us, 98 now; the 2816-wide one of 256 tokens 183, 150; the 8B's QKV of 512
 // tokens as 288 workgroups on 256 CUs, its 512-token turn 20.4 ms, 19.8 now).
+// The slots are an XCD's: 84 units of 3 token tiles fit the chip's 256, but four
+// XCDs get 11 units, 33 workgroups on 32 CUs (the 7168 x 5120 QKV of 384 tokens in
+// 3 splits 105 us, in 2 77).
 struct WidePlan {
     int tt, rows, ntt, ks;
 };
@@ -482,10 +485,13 @@ static WidePlan wide_plan(int64_t rows, int M, int nb, int cus, int mode) {
     p.tt = need <= 2 ? 2 : need <= 4 ? need : need <= 6 ? 6 : 8;
     p.ntt = (M + 16 * p.tt - 1) / (16 * p.tt);
     p.rows = (p.tt > 3 ? 256 : 128) / (mode == W_GLU ? 2 : 1);
-    const int64_t wgs = ((rows + p.rows - 1) / p.rows) * p.ntt, slots = (p.tt > 3 ? 1 : 2) * (int64_t)cus;
-    const int ks = (int)std::max<int64_t>(1, std::min<int64_t>({16, slots / wgs, (int64_t)nb / 2}));
-    const int per = std::max(1, (nb + ks - 1) / ks);
-    p.ks = std::max(1, (nb + per - 1) / per);  // no split without blocks
+    const int64_t tiles = (rows + p.rows - 1) / p.rows, slots = (p.tt > 3 ? 1 : 2) * (int64_t)cus;
+    auto whole = [&](int64_t ks) {  // no split without blocks
+        const int per = std::max<int>(1, (int)((nb + ks - 1) / ks));
+        return std::max(1, (nb + per - 1) / per);
+    };
+    p.ks = whole(std::max<int64_t>(1, std::min<int64_t>({16, slots / (tiles * p.ntt), (int64_t)nb / 2})));
+    while (p.ks > 1 && (tiles * p.ks + 7) / 8 * p.ntt > slots / 8) p.ks = whole(p.ks - 1);
     return p;
 }
 int wide_splits(int64_t rows, int M, int nb, int cus, int mode) { return wide_plan(rows, M, nb, cus, mode).ks; }
