@@ -123,3 +123,54 @@ def test_prompt_matmul_splits_fit_every_xcd():
                     many += ks > 1
                     assert ks == 1 or -(-units // 8) * ntt <= (32 if tt > 3 else 64), (glu, nb, rows, M, ks)
     assert many > 1000
+
+
+def test_prompt_attention_partials_bound():
+    """attn_prefill_partial_bytes bounds every launch of up to nq queries and max_keys keys: query blocks of
+    128 / G queries times the KV heads are a split's workgroups, a launch starts from 512 / workgroups splits of
+    at least 256 keys, 16 at most, and takes fewer, longer ones where that saves a round. And it is no more than twice
+    what some launch needs."""
+    bound = ts5hip.lib()._ZN6ts5hip26attn_prefill_partial_bytesEiiiil
+    bound.argtypes, bound.restype = [ctypes.c_int] * 4 + [ctypes.c_int64], ctypes.c_size_t
+
+    def splits(keys, wg):
+        want = max(256, -(-keys // max(1, min(16, -(-512 // wg)))))
+        first = -(-want // 64) * 64
+        best = None
+        for per in range(first, 2 * first + 1, 64):
+            n = -(-keys // per)
+            rounds = per + (0 if wg * n <= 512 else keys - (n - 1) * per if wg * (n - 1) <= 512 else per)
+            if best is None or rounds < best[0]:
+                best = rounds, n
+        return best[1]
+
+    for H, HKV, HD in ((32, 8, 128), (64, 8, 128), (40, 8, 128), (14, 2, 64), (8, 8, 128), (4, 1, 128)):
+        for keys in (256, 257, 600, 2048, 4096, 32768):
+            need = 0
+            for nq in sorted({*range(1, 513, 29), *range(32, 513, 32), *range(25, 513, 25), 512}):
+                n = splits(keys, -(-nq // (128 // (H // HKV))) * HKV)
+                need = max(need, nq * n * H * (HD + 4) * 4 if n > 1 else 0)
+                assert need <= bound(nq, H, HKV, HD, keys), (H, HKV, nq, keys)
+            assert bound(512, H, HKV, HD, keys) <= 2 * need, (H, HKV, keys)
+
+
+def test_fixed_memory_follows_the_buffers(tmp_path):
+    """The bytes beside the KV cache that a context is fitted into: the weights, the 512-token buffers with the
+    scratch of their matmuls and attention (64 query heads here), 256 logits rows with their picks, 64 MiB."""
+    import gguf_writer
+    hp = dict(synth.TINY_LLAMA, n_vocab=151936, n_layer=1, n_head=64, n_head_kv=8, head_dim=128)
+    tensors = {name: (t, ne0, ne1, np.zeros(synth.row_bytes(t, ne0) * ne1 if t else 4 * ne0 * ne1, np.uint8))
+               for name, t, ne0, ne1 in synth.tensor_specs(dict(hp, head_type=None))}
+    path = str(tmp_path / "m.gguf")
+    gguf_writer.write(path, gguf_writer.model_kv(hp, vocab_pieces=False), tensors)
+    fixed = ts5hip.gguf_hparams(path)[2]
+    weights = sum(ts5hip.lib().ts5hip_weight_bytes(t, ne0, ne1) if t else 4 * ne0 for t, ne0, ne1, _ in tensors.values())
+    E, F, AH, QR, V = 512, 1536, 64 * 128, 80 * 128, 151936
+    gemm = ts5hip.lib()._ZN6ts5hip18gemm_scratch_bytesElii
+    gemm.argtypes, gemm.restype = [ctypes.c_int64, ctypes.c_int, ctypes.c_int], ctypes.c_size_t
+    part = ts5hip.lib()._ZN6ts5hip26attn_prefill_partial_bytesEiiiil
+    part.argtypes, part.restype = [ctypes.c_int] * 4 + [ctypes.c_int64], ctypes.c_size_t
+    buffers = 4 * 512 * (2 * E + QR + 2 * AH + F) + 512 * 4 * AH
+    buffers += max(gemm(rows, M, ne0 // 256) for M in range(1, 513) for rows, ne0 in ((QR, E), (E, AH), (F, E), (E, F), (V, E)))
+    buffers += part(512, 64, 8, 128, 2 ** 31 - 1)
+    assert buffers <= fixed - weights <= buffers + 256 * 4 * V + (110 << 20)

@@ -484,11 +484,18 @@ static int pf_split_keys(int64_t max_keys, int64_t wg) {
     return (int)best;
 }
 
-// A bound for every launch with at most max_keys keys (splits <= 16 and
-// <= max_keys / 256, both growing with the key count).
-size_t attn_prefill_partial_bytes(int nq, int H, int HD, int64_t max_keys) {
-    const int64_t ns = std::min<int64_t>(16, (max_keys + 255) / 256);
-    return ns > 1 ? (size_t)nq * H * ns * (HD + 4) * sizeof(float) : 0;
+// A bound for every launch of at most nq queries over at most max_keys keys: no
+// more splits than pf_split_keys starts from, and those fall as the query blocks
+// grow (of 32/8 heads 512 queries take 4 splits, 128 take 16; 2400 rows of
+// partials at most).
+size_t attn_prefill_partial_bytes(int nq, int H, int HKV, int HD, int64_t max_keys) {
+    const int qb = PF_ROWS / (H / HKV);
+    int64_t most = 0;
+    for (int64_t blocks = 1; blocks <= (nq + qb - 1) / qb; blocks++) {
+        const int64_t ns = std::min<int64_t>({16, (512 + blocks * HKV - 1) / (blocks * HKV), (max_keys + 255) / 256});
+        if (ns > 1) most = std::max(most, std::min<int64_t>(nq, blocks * qb) * ns);
+    }
+    return (size_t)most * H * (HD + 4) * sizeof(float);
 }
 
 hipError_t launch_attn_prefill(const float *q, int64_t q_stride, KvLayer kv, int kv_f16, int n_ctx, int H, int HKV,

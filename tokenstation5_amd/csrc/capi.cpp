@@ -435,7 +435,8 @@ static int attn_prompt_into(ts5hip_ctx *ctx, const float *q, int nq, int n_head,
         return fail(ctx, TS5HIP_ERR_UNSUPPORTED, "prompt attention for %d/%d heads of %d", n_head, n_head_kv, head_dim);
     if (nq <= 0 || pos0 < 0 || n_ctx <= 0 || (int64_t)pos0 + nq > n_ctx)
         return fail(ctx, TS5HIP_ERR_ARG, "%d queries at %d in a cache of %d", nq, pos0, n_ctx);
-    if (int rc = ensure_scratch(ctx, attn_prefill_partial_bytes(nq, n_head, head_dim, (int64_t)pos0 + nq))) return rc;
+    if (int rc = ensure_scratch(ctx, attn_prefill_partial_bytes(nq, n_head, n_head_kv, head_dim, (int64_t)pos0 + nq)))
+        return rc;
     const KvLayer kv{(int8_t *)k, (uint16_t *)ks, (int8_t *)v, (uint16_t *)vs};
     TS5_HIP(ctx, launch_attn_prefill(q, (int64_t)n_head * head_dim, kv, kv_f16, n_ctx, n_head, n_head_kv, head_dim,
                                      pos0, nq, scale, (float *)ctx->scratch, out, ctx->stream));

@@ -68,6 +68,20 @@ inline size_t attn_partial_bytes(int B, int n_split, int H, int HKV, int HD) {
     return (size_t)B * n_split * HKV * attn_group_floats(H / HKV, HD) * sizeof(float);
 }
 
+// The buffers of several tokens per call (prompt passes, verify batches): the
+// activations, and the scratch that the largest of any token count of a pass
+// takes, for a model whose matrices have these types and shapes (model.cpp).
+struct MatShape {
+    uint32_t type;
+    int64_t ne0, ne1;
+};
+struct BatchSizes {
+    size_t x, qkv, q, att, ffn, otmp;      // floats
+    size_t act, gemm, part, counters;      // bytes
+    size_t bytes() const { return 4 * (x + qkv + q + att + ffn + otmp) + act + gemm + part + counters; }
+};
+BatchSizes batch_sizes(const ts5hip_hparams &hp, const std::vector<MatShape> &mats, int64_t n_ctx, bool kv_f16, int n_cu);
+
 // The draw of Engine::sample (engine/src/engine.cpp:34-45) from k candidates
 // sorted by descending logit: weights exp((l - l0) / T) in double, the
 // shortest prefix whose cumulative share reaches top_p, then

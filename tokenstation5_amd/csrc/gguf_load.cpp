@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "common_host.h"
+#include "kernels.h"
 #include "runtime.h"
 
 using namespace ts5hip;
@@ -280,18 +281,23 @@ bool hparams_of(const GgufFile &g, ts5hip_hparams &hp, int &n_ctx_train, std::st
 }
 
 // Bytes the model takes in HBM besides its KV cache: the weights in their HBM
-// layouts, the single-token buffers, and the 512-token batch buffers with the
-// logits rows.
-uint64_t fixed_bytes(const GgufFile &g, const ts5hip_hparams &hp) {
+// layouts, the buffers of several tokens per call, 256 logits rows with their
+// picks (the reference's logits capacity, engine/src/vk_backend.cpp:272-277) and 64
+// MiB for the rest (a token's buffers, the RoPE table).
+uint64_t fixed_bytes(const GgufFile &g, const ts5hip_hparams &hp, int n_cu) {
     uint64_t w = 0;
+    std::vector<MatShape> mats;
+    const int64_t QR = (int64_t)(hp.n_head + 2 * hp.n_head_kv) * hp.head_dim;
     for (const TensorInfo &t : g.tensors) {
         const int64_t rows = t.ne[1] * t.ne[2] * t.ne[3];
         const size_t db = device_bytes(t.type, t.ne[0], rows);
         w += db ? db : (uint64_t)t.ne[0] * rows * 4;
+        if (rows < 2) continue;
+        mats.push_back({device_type(t.type), t.ne[0], rows});
+        if (t.name.find("attn_q.weight") != std::string::npos) mats.push_back({device_type(t.type), t.ne[0], QR});
     }
-    const uint64_t T = 512, E = hp.n_embd, F = hp.n_ff, QR = (uint64_t)(hp.n_head + 2 * hp.n_head_kv) * hp.head_dim;
-    const uint64_t act = 4 * T * (2 * E + QR + 2ull * hp.n_head * hp.head_dim + F) + 2 * 4 * T * hp.n_vocab;
-    return w + act + (256ull << 20);  // plus scratch: matmul partials, attention partials, top-k
+    const uint64_t rows = 256ull * 4 * hp.n_vocab + topk_scratch_bytes(256);
+    return w + batch_sizes(hp, mats, INT32_MAX, false, n_cu).bytes() + rows + (64ull << 20);
 }
 
 }  // namespace
@@ -320,7 +326,7 @@ int ts5hip_gguf_hparams(const char *path, ts5hip_hparams *hp, int *n_ctx_train, 
     int train = 0;
     if (!parse(path, g, err) || !hparams_of(g, *hp, train, err)) return fail(nullptr, TS5HIP_ERR_ARG, "%s", err.c_str());
     if (n_ctx_train) *n_ctx_train = train;
-    if (fixed) *fixed = (int64_t)fixed_bytes(g, *hp);
+    if (fixed) *fixed = (int64_t)fixed_bytes(g, *hp, 256);  // (an MI355X's CUs)
     return TS5HIP_OK;
 }
 
@@ -347,7 +353,7 @@ int ts5hip_model_load(ts5hip_ctx *ctx, const char *path, int n_ctx, int kv_type,
         TS5_HIP(ctx, hipSetDevice(ctx->device));
         TS5_HIP(ctx, hipMemGetInfo(&free_b, &total_b));
         const int cap = train > 0 ? train : 32768;
-        const uint64_t used = fixed_bytes(g, hp);
+        const uint64_t used = fixed_bytes(g, hp, ctx->n_cu);
         const int f16 = ts5hip_fit_context(free_b, used, ts5hip_kv_bytes_per_token(&hp, KV_F16), cap);
         if (kv_type == KV_Q8 && ts5hip_f16_reaches(f16, cap)) kv_type = KV_F16;
         n_ctx = kv_type == KV_F16 ? f16 : ts5hip_fit_context(free_b, used, ts5hip_kv_bytes_per_token(&hp, KV_Q8), cap);

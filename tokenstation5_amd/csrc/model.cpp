@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -724,35 +725,22 @@ int ensure_batch(ts5hip_model *m) {
     if (m->bx) return TS5HIP_OK;
     const ts5hip_hparams &hp = m->hp;
     const int64_t E = hp.n_embd, F = hp.n_ff, AH = (int64_t)hp.n_head * hp.head_dim, QR = m->qkv_rows();
-    const int64_t wide = std::max({E, F, AH});
-    size_t gemm = 0, part = 0;
     const DevT &out = m->output.set ? m->output : m->tok_embd;
-    for (int M = 1; M <= CHUNK; M++) {
-        auto g = [&](int64_t rows, int64_t ne0, uint32_t t) {
-            const int bv = block_values(t) ? block_values(t) : 32;
-            gemm = std::max(gemm, gemm_scratch_bytes(rows, M, (int)(ne0 / bv)));
-        };
-        for (const LayerDev &L : m->layers) {
-            g(QR, E, L.qkv.type), g(E, AH, L.wo.type), g(F, E, L.gate.type), g(E, F, L.down.type);
+    std::vector<MatShape> mats{{out.type, E, hp.n_vocab}};
+    for (const LayerDev &L : m->layers) {
+        mats.insert(mats.end(), {{L.qkv.type, E, QR}, {L.wo.type, AH, E}, {L.gate.type, E, F}, {L.down.type, F, E}});
+        if (!L.in_qkv[0] || !L.in_qkv[1] || !L.in_qkv[2])
             for (int p = 0; p < 3; p++)
-                if (L.part[p].set) g(QR, E, L.part[p].type);
-        }
-        g(hp.n_vocab, E, out.type);
-        part = std::max(part, attn_partial_bytes(M, attn_splits(M, hp.n_head_kv, m->ctx->n_cu), hp.n_head, hp.n_head_kv, hp.head_dim));
-        if (attn_mq_fits(M, hp.n_head, hp.n_head_kv, hp.head_dim, m->kv_f16(), 0))
-            part = std::max(part, attn_partial_bytes(M, attn_mq_splits(hp.n_head_kv, m->ctx->n_cu), hp.n_head,
-                                                     hp.n_head_kv, hp.head_dim));
+                mats.push_back({L.in_qkv[p] ? L.qkv.type : L.part[p].type, E, p ? (int64_t)hp.n_head_kv * hp.head_dim : AH});
     }
-    part = std::max(part, attn_prefill_partial_bytes(CHUNK, hp.n_head, hp.head_dim, m->n_ctx));
+    const BatchSizes z = batch_sizes(hp, mats, m->n_ctx, m->kv_f16(), m->ctx->n_cu);
     int rc = 0;
-    if ((rc = alloc_t(m, CHUNK * E, &m->bx)) || (rc = alloc_t(m, CHUNK * QR, &m->bqkv)) ||
-        (rc = alloc_t(m, CHUNK * AH, &m->bq)) || (rc = alloc_t(m, CHUNK * AH, &m->batt)) ||
-        (rc = alloc_t(m, CHUNK * F, &m->bffn)) || (rc = alloc_t(m, CHUNK * E, &m->botmp)) ||
-        (rc = alloc(m, CHUNK * std::max({act_bytes(wide), mact_bytes(wide), hact_bytes(wide)}), &m->bact)) ||
-        (rc = alloc(m, std::max<size_t>(gemm, 256), &m->bgemm)) || (rc = alloc(m, part, (void **)&m->bpart)) ||
-        (rc = alloc_t(m, (size_t)CHUNK * hp.n_head_kv * CTR_STRIDE, &m->bcounters)))
+    if ((rc = alloc_t(m, z.x, &m->bx)) || (rc = alloc_t(m, z.qkv, &m->bqkv)) || (rc = alloc_t(m, z.q, &m->bq)) ||
+        (rc = alloc_t(m, z.att, &m->batt)) || (rc = alloc_t(m, z.ffn, &m->bffn)) || (rc = alloc_t(m, z.otmp, &m->botmp)) ||
+        (rc = alloc(m, z.act, &m->bact)) || (rc = alloc(m, z.gemm, &m->bgemm)) || (rc = alloc(m, z.part, (void **)&m->bpart)) ||
+        (rc = alloc(m, z.counters, (void **)&m->bcounters)))
         return rc;
-    TS5_HIP(m->ctx, hipMemsetAsync(m->bcounters, 0, (size_t)CHUNK * hp.n_head_kv * CTR_STRIDE * 4, m->ctx->stream));
+    TS5_HIP(m->ctx, hipMemsetAsync(m->bcounters, 0, z.counters, m->ctx->stream));
     return TS5HIP_OK;
 }
 
@@ -999,6 +987,26 @@ int run_tokens(ts5hip_model *m, const int32_t *tokens, int n, int pos0, bool wan
 }  // namespace
 
 namespace ts5hip {
+BatchSizes batch_sizes(const ts5hip_hparams &hp, const std::vector<MatShape> &mats, int64_t n_ctx, bool kv_f16, int n_cu) {
+    const int64_t E = hp.n_embd, F = hp.n_ff, AH = (int64_t)hp.n_head * hp.head_dim;
+    const int64_t QR = AH + 2ll * hp.n_head_kv * hp.head_dim, wide = std::max({E, F, AH});
+    std::set<std::pair<int64_t, int>> shapes;  // (rows, blocks a row)
+    for (const MatShape &t : mats) shapes.insert({t.ne1, (int)(t.ne0 / (block_values(t.type) ? block_values(t.type) : 32))});
+    size_t gemm = 256, part = 0;
+    for (int M = 1; M <= CHUNK; M++) {
+        for (const auto &t : shapes) gemm = std::max(gemm, gemm_scratch_bytes(t.first, M, t.second));
+        part = std::max(part, attn_partial_bytes(M, attn_splits(M, hp.n_head_kv, n_cu), hp.n_head, hp.n_head_kv, hp.head_dim));
+        if (attn_mq_fits(M, hp.n_head, hp.n_head_kv, hp.head_dim, kv_f16, 0))
+            part = std::max(part, attn_partial_bytes(M, attn_mq_splits(hp.n_head_kv, n_cu), hp.n_head, hp.n_head_kv, hp.head_dim));
+    }
+    if (attn_prefill_supported(hp.n_head, hp.n_head_kv, hp.head_dim))
+        part = std::max(part, attn_prefill_partial_bytes(CHUNK, hp.n_head, hp.n_head_kv, hp.head_dim, n_ctx));
+    const size_t T = CHUNK;
+    return BatchSizes{T * E, T * QR, T * AH, T * AH, T * F, T * E,
+                      T * std::max({act_bytes(wide), mact_bytes(wide), hact_bytes(wide)}), gemm, part,
+                      T * hp.n_head_kv * CTR_STRIDE * 4};
+}
+
 int model_vocab(const ts5hip_model *m) { return m->hp.n_vocab; }
 ts5hip_ctx *model_ctx(const ts5hip_model *m) { return m->ctx; }
 
