@@ -208,8 +208,8 @@ def test_long_prompt_logits_and_greedy_match_oracle(ctx, name):
 
 
 def test_prompt_chunks_split_at_512_and_256(ctx):
-    """Prompts go 512 tokens a pass, then 256, then the rest: one 1100-token call (512 + 512 + 76) against
-    the same tokens in calls of 700 (512 + 188) and 400 (256 + 144), and both against the oracle's last row.
+    """Prompts go 512 tokens a pass, then the rest: one 1100-token call (512 + 512 + 76) against
+    the same tokens in calls of 700 (512 + 188) and 400 (one pass), and both against the oracle's last row.
     The two GPU runs' sums run in other orders and can land q8 keys a step apart: the rows are held to the
     bar of the prompt test above, against the oracle."""
     hp, tensors, m = load(ctx, "tiny_llama_c", 1200)

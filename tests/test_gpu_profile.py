@@ -94,3 +94,17 @@ def test_profile_per_kernel(ctx, monkeypatch, graphs):
     assert sum(v[0] for v in pf.values()) <= total * 1.01 + 0.05
     assert m.take_profile() == ""
     m.close()
+
+
+def test_prompt_passes(ctx, monkeypatch):
+    """A call's tokens go 512 a pass while as many are left, and the rest in one pass, or as 256 and up to 64
+    where 257 to 320 are left: one embedding launch a pass."""
+    monkeypatch.setenv("TS5_PROFILE", "1")
+    m = ts5hip.Model(ctx, HP, 1200)
+    m.set_tensors(synth.model_tensors(HP, 21))
+    for n, passes in ((256, 1), (257, 2), (320, 2), (321, 1), (400, 1), (511, 1), (512, 1), (700, 2), (800, 3), (900, 2),
+                      (1100, 3)):
+        m.forward((np.arange(n) * 7 % HP["n_vocab"]).astype(np.int32), 0, logits=False)
+        pf, _ = parse(m.take_profile())
+        assert pf["embed_q4_k token_embd"][1] == passes, (n, pf["embed_q4_k token_embd"])
+    m.close()

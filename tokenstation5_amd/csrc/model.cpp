@@ -710,16 +710,22 @@ int host_rows_ready(ts5hip_model *m) {
 // Positions pos0.. of n tokens; logits rows (all or the last) left at
 // dev_rows / host_rows when want_logits.
 // Tokens per batched pass: the reference chunks prompts at 256 tokens
-// (engine/src/vk_backend.cpp:272-277), and logits_view holds 256 rows. Here 512
-// at a time while as many are left: twice the row and token tiles take half the
-// splits of K (the partial sums of an 8B layer's QKV, wo and down are 2 x 92 MB
-// of traffic a 256-token pass, 2 x 46 MB per 256 tokens of a 512-token one) and
-// half the key splits of the attention, and the small launches are shared: the
-// 8B's 512-token turn at 3584 cached tokens 22.4 -> 20.8 ms.
-// A rest below 512 goes as 256 and what is left: 300 tokens in one pass would
-// take three 128-token tiles, a second round of workgroups on a third of the CUs.
-constexpr int CHUNK = 512, HALF_CHUNK = 256;
-inline int chunk_tokens(int left) { return left >= CHUNK ? CHUNK : std::min(HALF_CHUNK, left); }
+// (engine/src/vk_backend.cpp:272-277), and logits_view holds 256 rows. Here up
+// to 512 at a time: twice the row and token tiles take half the splits of K (the
+// partial sums of an 8B layer's QKV, wo and down are 2 x 92 MB of traffic a
+// 256-token pass, 2 x 46 MB per 256 tokens of a 512-token one) and half the key
+// splits of the attention, and the small launches are shared: the 8B's 512-token
+// turn at 3584 cached tokens 22.4 -> 20.8 ms.
+// Fewer go in one pass too, but for 257 to 320: as 256 and a rest of at most 64, whose
+// matmuls run in small token tiles, where one pass would take three tiles of 96 to
+// 128 tokens. In ms, split against one pass, an 8B over a q8 cache: 257 tokens 11.6
+// and 12.9, 300 14.5 and 14.8, 320 15.1 and 15.0, 340 16.0 and 15.1, 384 16.9 and 15.5,
+// 511 19.9 and 16.9 (512 in one pass 16.9); the 48x5120 target 300 tokens 25.5 and 26.9,
+// 340 28.1 and 27.4; the 0.5B draft 300 8.4 and 6.2, 511 11.2 and 8.2.
+constexpr int CHUNK = 512, HALF_CHUNK = 256, SMALL_REST = 64;
+inline int chunk_tokens(int left) {
+    return left > HALF_CHUNK && left <= HALF_CHUNK + SMALL_REST ? HALF_CHUNK : std::min(CHUNK, left);
+}
 
 int ensure_batch(ts5hip_model *m) {
     if (m->bx) return TS5HIP_OK;
