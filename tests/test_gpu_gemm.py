@@ -107,11 +107,32 @@ def test_matmul_norm_and_accumulate(ctx):
 @pytest.mark.parametrize("ne0,rows", [(256, 1), (768, 130), (2304, 515)])
 def test_q4k_wide_matmul_edges(ctx, ne0, rows, ntok):
     """The prompt matmul at the edges of its token tiles (16-token groups of 2, 3, 4, 6, 8 a tile, one
-    token more), row tiles (128 and 256 rows, GLU half), splits of K down to one block, and rows that are
+    token more), row tiles (128 and 256 rows, GLU half), one split and three of three blocks, and rows that are
     no whole float4: store, accumulate and gate/up, each value against float64. The inputs are rounded to 22
     bits and the 32-bit sums run over at most 2304 products: 2e-5 of the row as in the tests above."""
     rng = np.random.default_rng(ne0 + 7 * rows + ntok)
     Wg, Wu = (synth.tensor(synth.Q4_K, ne0, rows, s, f"edge{ne0}_{rows}", centered=True) for s in (8, 9))
+    x = rng.standard_normal((ntok, ne0)).astype(np.float32)
+    y0 = rng.standard_normal((ntok, rows)).astype(np.float32)
+    wg, wu = (ctx.weight(synth.Q4_K, ne0, rows, w) for w in (Wg, Wu))
+    dx, y, h = ctx.to_device(x), ctx.to_device(y0), ctx.alloc(ntok * rows * 4)
+    want = oracle.matmul(synth.Q4_K, Wg, ne0, x)
+    got = run_matmul(ctx, synth.Q4_K, Wg, ne0, rows, x)
+    assert rel_l2(got, want) <= 2e-5
+    ctx.matmul(synth.Q4_K, wg, ne0, rows, dx, ntok, y, accumulate=True)
+    np.testing.assert_array_equal(y.download(np.float32, (ntok, rows)), y0 + got.reshape(ntok, rows))
+    ctx.matmul_glu(synth.Q4_K, wg, wu, ne0, rows, dx, ntok, h)
+    glu = oracle.swiglu(want, oracle.matmul(synth.Q4_K, Wu, ne0, x))
+    assert rel_l2(h.download(np.float32, (ntok, rows)), glu) <= 5e-5
+
+
+@pytest.mark.parametrize("ne0,rows,ntok", [(1792, 130, 17), (1792, 130, 48), (1792, 130, 128), (1792, 515, 200),
+                                            (13824, 128, 20), (13824, 130, 64), (13824, 515, 257)])
+def test_q4k_wide_matmul_uneven_splits(ctx, ne0, rows, ntok):
+    """Splits of K whose last is shorter: 7 blocks as 3, 3 and 1 (a split whose first block is its last), 54 as 13 of
+    4 and 2. Store, accumulate and gate/up against float64: inputs rounded to 22 bits and 32-bit sums, as above."""
+    rng = np.random.default_rng(ne0 + rows + ntok)
+    Wg, Wu = (synth.tensor(synth.Q4_K, ne0, rows, s, f"uneven{ne0}_{rows}", centered=True) for s in (8, 9))
     x = rng.standard_normal((ntok, ne0)).astype(np.float32)
     y0 = rng.standard_normal((ntok, rows)).astype(np.float32)
     wg, wu = (ctx.weight(synth.Q4_K, ne0, rows, w) for w in (Wg, Wu))

@@ -224,6 +224,41 @@ def test_prompt_chunks_split_at_512_and_256(ctx):
         assert err.max() <= 2e-3 and cos.min() > 0.999, (err.max(), cos.min())
 
 
+ONE = dict(n_layer=1, n_vocab=300)
+
+
+@pytest.mark.parametrize("hp,kv", [
+    (dict(synth.TINY_LLAMA_C, **ONE), ts5hip.KV_F16), (dict(synth.TINY_LLAMA_C, **ONE), ts5hip.KV_Q8),
+    (dict(synth.TINY_DRAFT_C, **ONE), ts5hip.KV_F16), (dict(synth.TINY_DRAFT_C, **ONE), ts5hip.KV_Q8),
+    (dict(synth.TINY_LLAMA_C, wtype=synth.Q6_K, **ONE), ts5hip.KV_F16),
+    (dict(synth.TINY_GEMMA3, n_layer=6, n_vocab=300, swa_window=200), ts5hip.KV_F16),
+    (dict(synth.TINY_GEMMA3, n_layer=6, n_vocab=300, swa_window=200, head_dim=128, n_head=8, n_head_kv=4), ts5hip.KV_Q8)])
+def test_512_token_passes_every_row(ctx, hp, kv):
+    """1100 tokens in one call (passes of 512, 512 and 76), then 400 in another (one pass), every position's
+    logits against the oracle's: Q4_K, Q8_0 and Q6_K matmuls, head dimensions 64 to 256, both caches, sliding
+    windows beside a global layer. One layer (six where a global one needs them) keeps rounding from growing: the
+    reference's bars of a whole model (engine/src/checks.cpp:145-159: 5e-3 of the largest over an f16 cache, 2e-2 over
+    q8). Over an f16 cache a key or value on a rounding edge can fall the other way, which these random weights can
+    turn into more (one row of the Q4_K model 8e-3, in calls of 100 tokens too): a row may also be off by as much as the
+    rounding of the whole cache moves it, the oracle's f16 cache against its f32 one."""
+    tensors = synth.model_tensors(hp, 31)
+    m = ts5hip.Model(ctx, hp, 1536, kv)
+    m.set_tensors(tensors)
+    ref = oracle.Model(hp, tensors, 1536, kv)
+    whole = oracle.Model(hp, tensors, 1536, ts5hip.KV_F32)
+    toks = np.array([(7 + 13 * i + (i * i) % 17) % hp["n_vocab"] for i in range(1500)], np.int32)
+    for a, b in ((0, 1100), (1100, 1500)):
+        got = m.forward(toks[a:b], a, all_logits=True)
+        want = ref.forward(toks[a:b], a, all_logits=True)
+        assert got.shape == want.shape == (b - a, hp["n_vocab"])
+        err, cos = row_errors(got, want)
+        bar = 2e-2
+        if kv == ts5hip.KV_F16:
+            bar = np.maximum(5e-3, row_errors(whole.forward(toks[a:b], a, all_logits=True), want)[0])
+        assert np.all(err <= bar) and cos.min() > 0.999, (a + err.argmax(), err.max(), cos.min())
+    m.close()
+
+
 def test_small_batches_wide_ffn_match_oracle(ctx):
     """Batches of 5, 3 and 1 tokens (the verify step's shapes) on a model whose
     ffn is wider than the fused matmul's LDS input (4608 > 4096): the gate/up
