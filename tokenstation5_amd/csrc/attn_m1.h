@@ -35,7 +35,7 @@
 // column a head. Per 16 keys a lane converts 8 scales instead of 32 and
 // splits 4 products into hi + lo instead of 16, about 100 of 330 vector
 // instructions less; these bound the kernel. 16 sequences of 24-32k keys, 32/8
-// heads: 224 -> 211 us (4.8 of the 5.2 TB/s that a copy reaches); a fourth step in
+// heads: 224 -> 209 us (4.8 of the 5.2 TB/s that a copy reaches); a fourth step in
 // flight changes nothing.
 #pragma once
 #include <type_traits>
@@ -210,16 +210,21 @@ __device__ inline void attn_m1(const AttnArgs &a, int split, int kvh, int b, int
                 R = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[c], R, 0, 0, 0);
             }
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                s[i] = R[i];
-                if constexpr (GC) {
-                    const float k = h2f(w.kg[i]);
-                    float x = R[i] * k;
-                    asm volatile("" : "+v"(x));
-                    x = fmaf(R[i], k, dpp_mov<0x128, 0xF>(x, x));  // row_ror:8: groups 0 + 2, 1 + 3,
-                    x = dpp_mov<0x128, 0xC>(x, x);                 // in columns 2 and 3 too
-                    s[i] = dpp_add<0x124, 0xF, true>(x);           // row_ror:4
-                }
+            for (int i = 0; i < 4; i++) s[i] = R[i];
+            if constexpr (GC) {  // step by step for all four: no row move waits for the one value before it
+                float k[4], x[4], y[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) k[i] = h2f(w.kg[i]), x[i] = R[i] * k[i];
+#pragma unroll
+                for (int i = 0; i < 4; i++) asm volatile("" : "+v"(x[i]));
+#pragma unroll
+                for (int i = 0; i < 4; i++) y[i] = dpp_mov<0x128, 0xF>(x[i], x[i]);  // row_ror:8
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[i] = fmaf(R[i], k[i], y[i]);  // groups 0 + 2, 1 + 3,
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[i] = dpp_mov<0x128, 0xC>(x[i], x[i]);  // in columns 2 and 3 too
+#pragma unroll
+                for (int i = 0; i < 4; i++) s[i] = dpp_add<0x124, 0xF, true>(x[i]);  // row_ror:4
             }
         } else {  // a sum per scale group, scaled
 #pragma unroll
