@@ -66,7 +66,7 @@ def decode_bench(ctx, hp, steps: int, warmup: int, prompt_len: int = PROMPT):
     prefill_s = time.time() - t0
     first = int(m.generate_greedy(int(prompt[-1]), prompt_len - 1, 1)[0])
     log(f"prefill of {prompt_len - 1} tokens: {prefill_s:.2f} s ({(prompt_len - 1) / prefill_s:.0f} tok/s, "
-        f"256-token batches)")
+        f"passes of up to 512 tokens)")
     if warmup:
         m.generate_greedy(first, prompt_len, warmup)
     ctx.sync()

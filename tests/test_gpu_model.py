@@ -162,8 +162,8 @@ def row_errors(got, want):
 
 @pytest.mark.parametrize("name", ["tiny_llama_c", "tiny_draft_c", "tiny_qwen3"])
 def test_long_prompt_logits_and_greedy_match_oracle(ctx, name):
-    """Prompts past 16 tokens take the prompt path. A 300-token prompt crosses
-    the 256-token chunk (engine/src/engine.cpp:172-183 is the reference's
+    """Prompts past 16 tokens take the prompt path. A 300-token prompt goes as 256
+    and 44 tokens (engine/src/engine.cpp:172-183 is the reference's
     256-token prompt loop); a second 37-token call at position 300 attends to
     keys it did not write. Every position's logits against the oracle's, then
     32 greedy tokens from the device loop against the oracle's host loop.

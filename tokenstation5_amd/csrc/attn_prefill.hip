@@ -47,9 +47,10 @@
 // The softmax's reference is the running maximum less 7, so that p goes to 128
 // and l and O carry the factor: a weight's lo plane leaves the fp16 subnormals
 // down to 2^-10 of the largest, not 2^-3 (700 keys with 2^-14.6 of the weight of
-// one without a value: 9.7e-5 from float64 before, 8e-6 at most now; 256 queries of normal
-// scores over 4096 keys 3.40e-7, 3.25e-7 now). Not more than 7: the reference is
-// rounded, and where its last place is 16, less 8 could become less 16 and p 2^16.
+// one without a value: 9.7e-5 from float64 before, 2.3e-6 now; 256 queries of
+// normal scores over 4096 keys 3.40e-7, 3.25e-7 now). Not more than 7: the
+// reference is rounded, and where its last place is 16, less 8 could become less
+// 16 and p 2^16.
 #include <algorithm>
 
 #include "common.h"
@@ -58,7 +59,6 @@
 namespace ts5hip {
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 

@@ -372,9 +372,10 @@ static int attn_decode_into(ts5hip_ctx *ctx, const float *q, int B, int n_head, 
     if (n_split <= 0) {
         n_split = attn_splits(B, n_head_kv, ctx->n_cu);
         // The multi-query kernel's work items hold all the batch's queries, so
-        // its splits fill the CUs by themselves (5 queries at 4101 keys, 32/8
-        // heads: 6 splits, 48 work items, 29 us; 32 splits 17 us), as many as
-        // the no-allocation scratch holds, so that both entry points agree.
+        // its splits fill the CUs by themselves, as a model's verify batches
+        // have them (5 queries at 4101 keys, 32/8 heads: 6 splits, 48 work items,
+        // 29 us; 32, of which 22 hold keys, 17 us), as many as the no-allocation
+        // scratch holds, so that both entry points agree.
         if (attn_mq_fits(B, n_head, n_head_kv, head_dim, kv_f16, kv_per_batch)) {
             const size_t one = attn_partial_bytes(B, 1, n_head, n_head_kv, head_dim);
             const int fit = (int)((NOALLOC_BYTES - NOALLOC_COUNTER_BYTES) / one);
