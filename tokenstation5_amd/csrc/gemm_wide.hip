@@ -48,9 +48,9 @@
 // the matrix core's time, at 2.2 GHz. It was twice that with the pieces read
 // right before their MFMAs. Gate/up of 256 tokens, 14336 x 4096: 152 us before
 // (64 of gate and up a 4-wave workgroup, two a CU, LDS reads and the unpack in
-// front of the MFMAs), 114 us now (527 TFLOP/s of useful products, twice that
-// issued); down 86 -> 57 us, QKV 54 -> 32 us, wo 37 -> 23 us, the last three
-// also by the outputs' way through LDS. 64 weight rows a wave (half the LDS
+// front of the MFMAs), 114-121 us now, run to run (497-527 TFLOP/s of useful
+// products, twice that issued); down 86 -> 57-59 us, QKV 54 -> 32-36 us, wo 37 ->
+// 23-24 us, the last three also by the outputs' way through LDS. 64 weight rows a wave (half the LDS
 // reads) measured slower: four waves of 64 rows x 128 tokens 138 us, eight of 64
 // x 64 151 us (their unpack is made twice, or no second wave hides the waits).
 #include <algorithm>
